@@ -673,9 +673,13 @@ def run_vision(reps: int = 5):
     rope_ms = med_ms(lambda: kernels.vision_rope_pad(qkv, run.pos_hw, run.cos, run.sin, h, hd, out=heads))
     rope_bytes = n * (3 * h * hd * 2 + 3 * h * kernels.HEAD_DIM * 2)
 
-    def attn(cu, plan):
-        return lambda: kernels.varlen_attention(heads[:, 0], heads[:, 1], heads[:, 2], cu, cu, hd ** -0.5,
-                                                causal=False, plan=plan, out=o, head_dim=run.attn_head_dim)
+    def window():  # rotary, attention and head layout of a window block in one launch
+        kernels.vision_window_attention(qkv, run.pos_hw, run.cos, run.sin, run.cu_window_host, run.cu_window, h,
+                                        hd ** -0.5)
+
+    def whole():
+        kernels.varlen_attention(heads[:, 0], heads[:, 1], heads[:, 2], run.cu_full, run.cu_full, hd ** -0.5,
+                                 causal=False, plan=run.plan_full, out=o, head_dim=run.attn_head_dim)
 
     out = {"workload": "Qwen2.5-VL vision tower (public config, random init), one 4K image: grid (1, 154, 274), "
                        "42196 patches -> 10549 tokens",
@@ -683,14 +687,14 @@ def run_vision(reps: int = 5):
            "rope_pad": {"ms": round(rope_ms, 4), "bytes": rope_bytes,
                         "gbps": round(rope_bytes / (rope_ms * 1e-3) / 1e9, 1),
                         "frac_hbm_peak": round(rope_bytes / (rope_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)}}
-    for name, cu_host, cu, plan in (("window_attention", lay.cu_window, run.cu_window, run.plan_window),
-                                    ("whole_image_attention", lay.cu_full, run.cu_full, run.plan_full)):
-        ms = med_ms(attn(cu, plan))
+    # bytes each moves at least: q, k and v read, the output written (whole image: 128-element head rows)
+    for name, cu_host, fn, row in (("window_attention", lay.cu_window, window, hd),
+                                   ("whole_image_attention", lay.cu_full, whole, kernels.HEAD_DIM)):
+        ms = med_ms(fn)
         pairs = sum((b - a) ** 2 for a, b in zip(cu_host, cu_host[1:]))
         tf = 4.0 * pairs * hd * h / (ms * 1e-3) / 1e12
-        # bytes the kernel moves at least: q, k and v head rows read (128-element rows), output written
-        nbytes = 4 * n * h * kernels.HEAD_DIM * 2
-        out[name] = {"ms": round(ms, 4), "sequences": len(cu_host) - 1, "work_items": plan.num_items,
+        nbytes = 4 * n * h * row * 2
+        out[name] = {"ms": round(ms, 4), "sequences": len(cu_host) - 1,
                      "kernel_head_dim": run.attn_head_dim, "tflops": round(tf, 1),
                      "frac_mfma_peak": round(tf / MFMA_BF16_PEAK_TFLOPS, 4),
                      "gbps": round(nbytes / (ms * 1e-3) / 1e9, 1),

@@ -301,6 +301,26 @@ int vlc_vision_rope_pad(const void* qkv, int64_t qkv_row_stride, const int32_t* 
                         void* out, int64_t out_row_stride, void* stream);
 
 /*
+ * Vision tower: the whole attention of a block that attends within windows, from the QKV
+ * projection's rows to the output projection's input: 2-D rotary of q and k (as
+ * vlc_vision_rope_pad), non-causal attention within each window, heads written unpadded.
+ * Replaces VisionAttention.forward between its projections (models/qwen2_5_vl.py:176-212).
+ *
+ * qkv, pos_hw, cos_table, sin_table, max_pos: as vlc_vision_rope_pad.
+ * cu_host / cu_dev: int32 [num_windows + 1] window boundaries in tokens, non-decreasing, in
+ *   host memory and as a device copy; at most 64 tokens a window (VLC_ERR_UNSUPPORTED
+ *   otherwise).  Tokens outside [cu[0], cu[num_windows]) are not written.
+ * head_dim: 80 (VLC_ERR_UNSUPPORTED otherwise).
+ * out: [num_tokens][num_heads][80] bf16 at row stride out_row_stride.
+ * qkv, out and their row strides 16-byte aligned, the tables 8-byte aligned.
+ */
+int vlc_vision_window_attn(const void* qkv, int64_t qkv_row_stride, const int32_t* pos_hw,
+                           const void* cos_table, const void* sin_table, int64_t max_pos,
+                           const int32_t* cu_host, const int32_t* cu_dev, int num_windows,
+                           int64_t num_tokens, int num_heads, int head_dim, float softmax_scale,
+                           void* out, int64_t out_row_stride, void* stream);
+
+/*
  * RMSNorm, optionally with the residual add fused in front of it.
  * Replaces RMSNorm.rms_forward / add_rms_forward (layers/layernorm.py:16-40),
  * used by the decoder (models/qwen3.py:145-158, :184) and the vision tower

@@ -302,3 +302,39 @@ def test_random_grids(dev, seed):
         ref = oattn.varlen_attention(hc[:, 0, :, :80], hc[:, 1, :, :80], hc[:, 2, :, :80], cu_h, cu_h,
                                      80 ** -0.5, False)
         assert_attn_close(o[..., :80], ref, what=f"random grids {grids}")
+
+
+@pytest.mark.parametrize("heads", [16, 6], ids=["16-heads", "6-heads"])
+@pytest.mark.parametrize("grids", [[(1, 2, 2)], [(1, 8, 8)], [(1, 10, 6), (2, 16, 18)], [(1, 22, 34)]],
+                         ids=["one-unit", "one-window", "ragged", "edges"])
+def test_window_attention_kernel(dev, grids, heads):
+    """vlc_vision_window_attn (rotary + window attention + head layout in one launch) against the
+    oracle's rotation and fp32 attention: windows of 4 to 64 patches, head counts off the
+    workgroup's four, qkv rows with a gap behind them.  Rounding: q, k and v are the oracle's own bf16
+    values, so the usual attention bar (tests/_util.py) holds."""
+    say(f"vision: window attention kernel grids={grids} heads={heads}")
+    lay, qkv, cos, sin = _rope_inputs(dev, grids, heads=heads, seed=17)
+    n = lay.num_patches
+    ph, pw = torch.from_numpy(lay.pos_hw[:, 0]).long(), torch.from_numpy(lay.pos_hw[:, 1]).long()
+    c, s = cos.cpu(), sin.cpu()
+    c80, s80 = torch.cat((c[ph], c[pw]) * 2, -1), torch.cat((s[ph], s[pw]) * 2, -1)
+    q, k, v = qkv.reshape(n, 3, heads, 80).unbind(1)
+    ref = oattn.varlen_attention(ov.rope_bf16(q, c80, s80), ov.rope_bf16(k, c80, s80), v, lay.cu_window,
+                                 lay.cu_window, 80 ** -0.5, False)
+    wide = torch.full((n, 3 * heads * 80 + 8), float("nan"), dtype=torch.bfloat16, device=dev)
+    wide[:, :-8] = qkv.to(dev)
+    cu = np.asarray(lay.cu_window, dtype=np.int32)
+    for rows in (qkv.to(dev), wide[:, :-8]):
+        o = kernels.vision_window_attention(rows, torch.from_numpy(lay.pos_hw).to(dev), cos, sin, cu,
+                                            torch.from_numpy(cu).to(dev), heads, 80 ** -0.5)
+        assert_attn_close(o.cpu().view(n, heads, 80), ref, what="window attention kernel")
+
+
+def test_window_attention_refuses_long_windows_and_bad_boundaries(dev):
+    """Host checks only: nothing is launched."""
+    lay, qkv, cos, sin = _rope_inputs(dev, [(1, 16, 16)])
+    pos = torch.from_numpy(lay.pos_hw).to(dev)
+    for bad, status in (([0, 65, 256], -2), ([0, 40, 30], -1), ([0, 64, 320], -1)):
+        cu = np.asarray(bad, dtype=np.int32)
+        with pytest.raises(RuntimeError, match=f"status {status}"):
+            kernels.vision_window_attention(qkv.to(dev), pos, cos, sin, cu, torch.from_numpy(cu).to(dev), 16, 0.1)

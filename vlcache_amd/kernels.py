@@ -539,6 +539,24 @@ def decode_attention_noalloc(q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
 
 
 # --------------------------------------------------------------------------- vision tower
+VISION_WINDOW_MAX = 64  # patches per window of vlc_vision_window_attn
+VISION_HEAD_DIM = 80    # its head_dim
+
+
+def _check_vision_rows(qkv, pos_hw, cos_table, sin_table, num_heads: int, head_dim: int) -> None:
+    n = qkv.shape[0]
+    if qkv.dtype != torch.bfloat16 or qkv.dim() != 2 or qkv.shape[1] != 3 * num_heads * head_dim or qkv.stride(1) != 1:
+        raise ValueError(f"qkv must be bf16 [N, {3 * num_heads * head_dim}] with contiguous rows")
+    if pos_hw.dtype != torch.int32 or tuple(pos_hw.shape) != (n, 2) or not pos_hw.is_contiguous():
+        raise ValueError("pos_hw must be contiguous int32 [N, 2]")
+    q4 = head_dim // 4
+    for name, t in (("cos_table", cos_table), ("sin_table", sin_table)):
+        if t.dtype != torch.bfloat16 or t.dim() != 2 or t.shape[1] != q4 or not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous bf16 [max_pos, {q4}]")
+    if cos_table.shape != sin_table.shape:
+        raise ValueError("cos_table and sin_table differ in shape")
+
+
 def vision_rope_pad(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.Tensor,
                     num_heads: int, head_dim: int, padded_dim: int = HEAD_DIM,
                     out: torch.Tensor | None = None) -> torch.Tensor:
@@ -551,16 +569,7 @@ def vision_rope_pad(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Te
     """
     _require_device("vision_rope_pad", qkv, pos_hw, cos_table, sin_table, out)
     n = qkv.shape[0]
-    if qkv.dtype != torch.bfloat16 or qkv.dim() != 2 or qkv.shape[1] != 3 * num_heads * head_dim or qkv.stride(1) != 1:
-        raise ValueError(f"qkv must be bf16 [N, {3 * num_heads * head_dim}] with contiguous rows")
-    if pos_hw.dtype != torch.int32 or tuple(pos_hw.shape) != (n, 2) or not pos_hw.is_contiguous():
-        raise ValueError("pos_hw must be contiguous int32 [N, 2]")
-    q4 = head_dim // 4
-    for name, t in (("cos_table", cos_table), ("sin_table", sin_table)):
-        if t.dtype != torch.bfloat16 or t.dim() != 2 or t.shape[1] != q4 or not t.is_contiguous():
-            raise ValueError(f"{name} must be contiguous bf16 [max_pos, {q4}]")
-    if cos_table.shape != sin_table.shape:
-        raise ValueError("cos_table and sin_table differ in shape")
+    _check_vision_rows(qkv, pos_hw, cos_table, sin_table, num_heads, head_dim)
     if out is None:
         out = torch.empty(n, 3, num_heads, padded_dim, dtype=torch.bfloat16, device=qkv.device)
     elif out.dtype != torch.bfloat16 or tuple(out.shape) != (n, 3, num_heads, padded_dim) or \
@@ -570,6 +579,31 @@ def vision_rope_pad(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Te
         qkv.data_ptr(), qkv.stride(0), pos_hw.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(),
         cos_table.shape[0], n, num_heads, head_dim, padded_dim, out.data_ptr(), out.stride(0), _stream(qkv))
     _lib.check("vlc_vision_rope_pad", st)
+    return out
+
+
+def vision_window_attention(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Tensor,
+                            sin_table: torch.Tensor, cu_host: np.ndarray, cu_dev: torch.Tensor, num_heads: int,
+                            softmax_scale: float) -> torch.Tensor:
+    """Rotary, attention within windows and head layout of one vision block (vlc_vision_window_attn).
+
+    qkv: [N, 3 * num_heads * 80] bf16 rows; pos_hw and the tables as vision_rope_pad; cu_host
+    (int32 numpy) and cu_dev (int32, device): the same window boundaries, at most
+    VISION_WINDOW_MAX tokens a window.  Returns [N, num_heads * 80] bf16.
+    """
+    _require_device("vision_window_attention", qkv, pos_hw, cos_table, sin_table, cu_dev)
+    _check_vision_rows(qkv, pos_hw, cos_table, sin_table, num_heads, VISION_HEAD_DIM)
+    if cu_host.dtype != np.int32 or cu_host.ndim != 1 or not cu_host.flags.c_contiguous or cu_host.size < 1:
+        raise ValueError("cu_host must be a contiguous int32 vector")
+    if cu_dev.dtype != torch.int32 or cu_dev.numel() != cu_host.size or not cu_dev.is_contiguous():
+        raise ValueError("cu_dev must be a contiguous int32 copy of cu_host")
+    n = qkv.shape[0]
+    out = torch.empty(n, num_heads * VISION_HEAD_DIM, dtype=torch.bfloat16, device=qkv.device)
+    st = _lib.load().vlc_vision_window_attn(
+        qkv.data_ptr(), qkv.stride(0), pos_hw.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(),
+        cos_table.shape[0], cu_host.ctypes.data, cu_dev.data_ptr(), cu_host.size - 1, n, num_heads,
+        VISION_HEAD_DIM, float(softmax_scale), out.data_ptr(), out.stride(0), _stream(qkv))
+    _lib.check("vlc_vision_window_attn", st)
     return out
 
 

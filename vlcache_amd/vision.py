@@ -132,6 +132,9 @@ class VisionAttention(nn.Module):
     def forward(self, x, run: "_Run", full: bool):
         n = x.shape[0]
         qkv = self.qkv(x)
+        if not full and run.fused_windows:
+            return self.proj(kernels.vision_window_attention(qkv, run.pos_hw, run.cos, run.sin, run.cu_window_host,
+                                                             run.cu_window, self.num_heads, self.head_dim ** -0.5))
         heads = kernels.vision_rope_pad(qkv, run.pos_hw, run.cos, run.sin, self.num_heads, self.head_dim)
         cu, plan = (run.cu_full, run.plan_full) if full else (run.cu_window, run.plan_window)
         o = kernels.varlen_attention(heads[:, 0], heads[:, 1], heads[:, 2], cu, cu, self.head_dim ** -0.5,
@@ -228,13 +231,18 @@ class VisionTransformer(nn.Module):
         cos, sin = self.rope_tables(lay.max_pos)
         # 80-dim heads have a kernel of their own; other widths run as zero-padded 128-dim heads
         ahd = self.head_dim if self.head_dim in kernels.ATTN_HEAD_DIMS else kernels.HEAD_DIM
-        run = _Run(layout=lay, attn_head_dim=ahd,
+        # windows of at most 64 patches with 80-dim heads run as one kernel per block
+        cu_window_host = np.asarray(lay.cu_window, dtype=np.int32)
+        fused = self.head_dim == kernels.VISION_HEAD_DIM and \
+            int(np.diff(cu_window_host).max(initial=0)) <= kernels.VISION_WINDOW_MAX
+        run = _Run(layout=lay, attn_head_dim=ahd, fused_windows=fused, cu_window_host=cu_window_host,
                    patch_order=torch.from_numpy(lay.patch_order).to(dev),
                    reverse=torch.from_numpy(lay.reverse).to(dev),
                    pos_hw=torch.from_numpy(lay.pos_hw).to(dev),
                    cos=cos, sin=sin,
                    cu_window=cu_t(lay.cu_window), cu_full=cu_t(lay.cu_full),
-                   plan_window=kernels.plan_attention(lay.cu_window, lay.cu_window, h, h, ahd, False, dev),
+                   plan_window=None if fused else
+                   kernels.plan_attention(lay.cu_window, lay.cu_window, h, h, ahd, False, dev),
                    plan_full=kernels.plan_attention(lay.cu_full, lay.cu_full, h, h, ahd, False, dev))
         self._runs[key] = run
         while len(self._runs) > self._plan_cache:
