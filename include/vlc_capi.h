@@ -369,6 +369,19 @@ int vlc_linear_skinny(const void* x, int64_t x_row_stride, int64_t rows, int64_t
                       const void* weight, int64_t w_row_stride, int64_t out_features, const void* bias,
                       void* out, int64_t out_row_stride, void* stream);
 
+/*
+ * The same for at most 64 rows, K split across workgroups (long K, few features: the down
+ * projection of a decode step with many sequences).  Operands as vlc_linear_skinny, with
+ * out_features a multiple of 32.  workspace: device scratch of at least
+ * vlc_linear_split_workspace(rows, out_features) bytes, 16-byte aligned, used by this call
+ * only; its contents before and after do not matter.
+ */
+int64_t vlc_linear_split_workspace(int64_t rows, int64_t out_features);
+int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
+                     const void* weight, int64_t w_row_stride, int64_t out_features, const void* bias,
+                     void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes,
+                     void* stream);
+
 #ifdef __cplusplus
 }
 #endif

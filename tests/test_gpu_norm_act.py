@@ -178,3 +178,45 @@ def test_random_shapes(dev, seed):
     ref = xs.float() @ ws.float().t() + (b.float() if b is not None else 0.0)
     tol = ref.abs() * 2.0 ** -7 + ref.abs().max() * k * 2.0 ** -24
     assert int(((y - ref).abs() > tol).sum()) == 0
+
+
+# The edges of the kernel choice: rows 1, 2 | 3, 4 | 5, 8 | 9, 16; K a multiple of 32 only, of 64, 128
+# and 256; N on each side of the tile-count lines and not a multiple of 32; a last workgroup with idle tiles.
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("k,n", [(32, 16), (96, 48), (64, 4480), (128, 3200), (256, 3216), (320, 12800), (2048, 12816)])
+def test_linear_skinny_kernel_choice(dev, m, k, n):
+    """One bf16 ulp of the fp32 product plus the reordering of K fp32 terms (the bar of test_linear_skinny)."""
+    from vlcache_amd import kernels
+
+    say(f"linear_skinny choice m={m} k={k} n={n}")
+    x, w, b = randn_bf16((m, k), m + k), randn_bf16((n, k), n + k, 0.05), randn_bf16((n,), 9)
+    out = kernels.linear_skinny(x.to(dev), w.to(dev), b.to(dev)).float().cpu()
+    ref = x.float() @ w.float().t() + b.float()
+    tol = ref.abs() * 2.0 ** -7 + ref.abs().max() * k * 2.0 ** -24
+    assert int(((out - ref).abs() > tol).sum()) == 0
+
+
+@pytest.mark.parametrize("m", [1, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("k,n,bias", [(32, 32, True), (2048, 512, True), (11008, 2048, False), (4128, 8224, False)])
+def test_linear_split(dev, m, k, n, bias):
+    """vlc_linear_split: row blocks' edges, fewer k steps than splits, one split only (N 8224), through
+    the layer too; the bar of test_linear_skinny."""
+    from vlcache_amd import kernels
+    from vlcache_amd.layers.linear import Linear
+
+    say(f"linear_split m={m} k={k} n={n} bias={bias}")
+    x, w = randn_bf16((m, k + 8), m + k)[:, :k], randn_bf16((n, k), n + k, 0.05)
+    b = randn_bf16((n,), 9) if bias else None
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev) if bias else None
+    out = kernels.linear_split(xd, wd, bd)
+    ref = x.float() @ w.float().t() + (b.float() if bias else 0.0)
+    tol = ref.abs() * 2.0 ** -7 + ref.abs().max() * k * 2.0 ** -24
+    assert int(((out.float().cpu() - ref).abs() > tol).sum()) == 0
+    if m > 16 and k >= 4 * n:
+        lin = Linear(k, n, bias=bias, device=dev, dtype=torch.bfloat16)
+        with torch.no_grad():
+            lin.weight.copy_(wd)
+            if bias:
+                lin.bias.copy_(bd)
+            assert torch.equal(lin(xd), out)
+        assert lin(xd).requires_grad  # with gradients on, the layer stays torch's

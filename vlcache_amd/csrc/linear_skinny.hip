@@ -1,25 +1,39 @@
-// Skinny linear layer for decode steps: out[m][n] = bf16( sum_k x[m][k] * w[n][k] + bias[n] )
-// for M <= 16 rows of x.
+// Linear layers of a few rows, for decode steps: out[m][n] = bf16(sum_k x[m][k] w[n][k] + bias[n]).
 //
-// In a decode step the projections of the decoder (models/qwen3.py: QKV, output,
-// gate/up and down projections, and the LM head) multiply a handful of token rows by
-// the whole weight matrix, so the work is streaming the weights from HBM once; the
-// library GEMMs reach about 2-3 TB/s on these shapes with cold weights.  A wave
-// owns a tile of 16 output features and a K range: it streams the range of the 16
-// weight rows (16 bytes per lane per 32-k step, U steps in flight) and multiplies
-// them with the matching x slice on the matrix pipe,
-//   C (16 features x 16 rows) += W (16 x 32) . X^T (32 x 16)   v_mfma_f32_16x16x32_bf16,
-// x rows >= M read as zero.  KS waves of a workgroup share a tile (K split KS ways);
-// their partial C tiles are summed through LDS in a fixed order, the bias is added in
-// fp32 and the result rounded to bf16 once.
+// In a decode step the projections of the decoder (models/qwen3.py: QKV, output, gate/up
+// and down projections, and the LM head) multiply a handful of token rows by the whole
+// weight matrix, so the work is streaming the weights from HBM once.
+//
+// A wave multiplies a 16-row tile of weights with 16 columns of x on the matrix pipe,
+// v_mfma_f32_16x16x32_bf16, 64 bytes of a weight row per instruction and row.  Few rows of
+// x leave most of the 16 columns empty, so the tile's 16 x 16 products are used as Z
+// diagonal blocks of 16 / Z features x 16 / Z rows, each block summing its own 32 of 32 Z
+// consecutive k: the tile then reads 64 Z contiguous bytes of each weight row (1 KB of two
+// rows for Z = 8) and there are Z times as many tiles to spread over the chip, which is
+// what shapes with few features lack.  TF tiles of features share each x operand, RB row
+// blocks each weight operand, KS waves of a workgroup split K; the partial products meet
+// in LDS in a fixed order, the bias is added in fp32 and the sum rounded to bf16 once.
+// The cost beside the weights is x, which every tile reads again from L2: 16 / (Z TF)
+// times fewer bytes per row for a larger tile.
+//
+// Measured, us, cold weights, calls of distinct weights in one graph, K x N; before is a
+// tile of Z = 1, TF = 1 with K split four or eight ways:
+//   rows                     3584 x 4608  3584^2  3584 x 37888  18944 x 3584  2048 x 22016  11008 x 2048
+//   1, Z 8 TF 1 (before)                                                      15.7 (19.6)   10.3 (20.7)
+//   4, Z 4 TF 2, 4 (before)  11.1 (12.9)  8.1 (8.5)  49.6 (54.3)  27.6 (28.6)  18.8 (20.5)   12.3 (20.7)
+//   8, Z 2 (Z 1)             12.4 (12.9)  8.9 (9.0)  52.5 (62)    30.0 (33)    20.6 (23)     13.7 (18)
+//   16, Z 1, or Z 2 RB 2     14.2         9.9        57.6 (75.8)  36.9         22.6 (25.3)   17.8
+// and, one row, 2048 x 2560 4.1 (5.2), 2048^2 3.7 (5.0), 2048 x 151936 95.9 (104.8).
+#include <type_traits>
+
 #include "common.h"
 
 namespace vlc {
 namespace {
 
-constexpr int kWaves = 8;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kMaxRows = 16;
+constexpr int kMaxRows = 16;       // vlc_linear_skinny
+constexpr int kMaxSplitRows = 64;  // vlc_linear_split
+constexpr int kPad = 17;           // floats per row of a 16 x 16 partial tile in LDS
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -29,80 +43,139 @@ __device__ __forceinline__ bf16x8 ld16(const char* p) {
   return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4v*>(p));
 }
 
-// KS waves split K for each 16-feature tile; a workgroup holds kWaves / KS tiles.
-template <int U, int KS>
-__global__ __launch_bounds__(kThreads) void linear_skinny_kernel(const char* __restrict__ x, int64_t x_stride_b,
-                                                                 int rows, int k_steps, int tiles,
-                                                                 const char* __restrict__ w, int64_t w_stride_b,
-                                                                 const uint16_t* __restrict__ bias,
-                                                                 uint16_t* __restrict__ out, int64_t out_stride) {
-  constexpr int kTiles = kWaves / KS;
-  __shared__ f32x4 part[KS > 1 ? kWaves : 1][64];
+struct Args {
+  const char* x;
+  int64_t x_stride_b;
+  int rows, k_steps, tiles;
+  const char* w;
+  int64_t w_stride_b;
+  const uint16_t* bias;
+  uint16_t* out;
+  int64_t out_stride;
+  float* partial;  // gridDim.y > 1: [gridDim.y][rows][out_features]
+  int out_features;
+};
+
+// U: k steps in flight; KS waves of the workgroup's W split K; gridDim.y splits it further.
+template <int U, int KS, int Z, int TF, int RB, int W>
+__global__ __launch_bounds__(64 * W) void linear_skinny_kernel(const Args p) {
+  constexpr int kTiles = W / KS;  // tiles of a workgroup
+  constexpr int F = 16 / Z;       // features, and rows, of a diagonal block
+  constexpr int kStepB = 64 * Z;  // bytes of a row per k step
+  __shared__ float part[W][TF][RB][16 * kPad];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int tile = wave / KS, ks = wave % KS;
-  const int r = lane & 15;              // A: feature row of the tile; B: row of x
-  const int kq = (lane >> 4) * 16;      // byte offset of the lane's 8 k values in a 32-k step
-  const int t = blockIdx.x * kTiles + tile;
-  const bool live = t < tiles;          // the last workgroup's tiles past N do no work
-  const int f0 = (live ? t : 0) * 16;
-  const char* wp = w + (int64_t)(f0 + r) * w_stride_b + kq;
-  const bool xr = r < rows;
-  const char* xp = x + (int64_t)(xr ? r : 0) * x_stride_b + kq;
-  // the wave's contiguous range of 32-k steps
-  const int per = (k_steps + KS - 1) / KS;
-  const int s0 = live ? min(k_steps, ks * per) : 0, s1 = live ? min(k_steps, s0 + per) : 0;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int r = lane & 15, g = lane >> 4;
+  const int z = r / F, f = r % F;  // diagonal block; feature (A) or row of x (B) within it
+  const int t = blockIdx.x * kTiles + wave / KS;
+  const bool live = t < p.tiles;   // the last workgroup's tiles past N do no work
+  const char* wp = p.w + (int64_t)((live ? t : 0) * (F * TF) + f) * p.w_stride_b + z * 64 + g * 16;
+  const char* xp[RB];
+  bool xr[RB];
+#pragma unroll
+  for (int q = 0; q < RB; ++q) {
+    const int m = f + F * q;
+    xr[q] = m < p.rows;  // other rows read as zero
+    xp[q] = p.x + (int64_t)(xr[q] ? m : 0) * p.x_stride_b + z * 64 + g * 16;
+  }
+  const int splits = KS * (int)gridDim.y, split = (int)blockIdx.y * KS + wave % KS;
+  int s = live ? (int)((int64_t)p.k_steps * split / splits) : 0;
+  const int s1 = live ? (int)((int64_t)p.k_steps * (split + 1) / splits) : 0;
   const bf16x8 zero = __builtin_bit_cast(bf16x8, u32x4v{0u, 0u, 0u, 0u});
-  int s = s0;
-  for (; s + U <= s1; s += U) {
-    bf16x8 a[U], b[U];
+  f32x4 acc[TF][RB] = {};
+  auto steps = [&](auto depth, int s0) __attribute__((always_inline)) {
+    constexpr int D = decltype(depth)::value;
+    bf16x8 a[D][TF], b[D][RB];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      a[u] = ld16(wp + (int64_t)(s + u) * 64);
-      b[u] = xr ? ld16(xp + (int64_t)(s + u) * 64) : zero;
+    for (int u = 0; u < D; ++u) {
+#pragma unroll
+      for (int j = 0; j < TF; ++j) a[u][j] = ld16(wp + (int64_t)(j * F) * p.w_stride_b + (int64_t)(s0 + u) * kStepB);
+#pragma unroll
+      for (int q = 0; q < RB; ++q) b[u][q] = xr[q] ? ld16(xp[q] + (int64_t)(s0 + u) * kStepB) : zero;
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
-  }
-  for (; s < s1; ++s) {
-    const bf16x8 a = ld16(wp + (int64_t)s * 64);
-    const bf16x8 b = xr ? ld16(xp + (int64_t)s * 64) : zero;
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-  }
-  if constexpr (KS > 1) {
-    if (ks > 0) part[wave][lane] = acc;
-    __syncthreads();
-    if (ks != 0) return;
+    for (int u = 0; u < D; ++u)
 #pragma unroll
-    for (int v = 1; v < KS; ++v) {
-      const f32x4 p = part[wave + v][lane];
-      acc[0] += p[0], acc[1] += p[1], acc[2] += p[2], acc[3] += p[3];
-    }
+      for (int j = 0; j < TF; ++j)
+#pragma unroll
+        for (int q = 0; q < RB; ++q)
+          acc[j][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][j], b[u][q], acc[j][q], 0, 0, 0);
+  };
+  for (; s + U <= s1; s += U) steps(std::integral_constant<int, U>{}, s);
+  for (; s < s1; ++s) steps(std::integral_constant<int, 1>{}, s);
+
+  // lane holds C[row 4 g + e][column r] of its tiles
+#pragma unroll
+  for (int j = 0; j < TF; ++j)
+#pragma unroll
+    for (int q = 0; q < RB; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part[wave][j][q][(4 * g + e) * kPad + r] = acc[j][q][e];
+  __syncthreads();
+  // output (tile, row block, row, feature) = sum over the waves of the tile and the diagonal blocks
+  constexpr int kOut = kTiles * RB * F * TF * F;
+  for (int i = threadIdx.x; i < kOut; i += 64 * W) {
+    const int ff = i % F, j = i / F % TF, m = i / (F * TF) % F, q = i / (F * TF * F) % RB, tt = i / (F * TF * F * RB);
+    const int row = m + F * q, tile = blockIdx.x * kTiles + tt;
+    if (row >= p.rows || tile >= p.tiles) continue;
+    float y = 0.f;
+#pragma unroll
+    for (int v = 0; v < KS; ++v)
+#pragma unroll
+      for (int zz = 0; zz < Z; ++zz) y += part[tt * KS + v][j][q][(zz * F + ff) * kPad + zz * F + m];
+    const int n = (tile * TF + j) * F + ff;
+    if (gridDim.y == 1)
+      p.out[row * p.out_stride + n] =
+          (uint16_t)f32_to_bf16_bits(p.bias ? y + bf16_bits_to_f32(p.bias[n]) : y);
+    else
+      p.partial[((int64_t)blockIdx.y * p.rows + row) * p.out_features + n] = y;
   }
-  // lane holds C[feature 4 (lane / 16) + t][row lane % 16], t = 0..3
-  const int m = lane & 15;
-  if (m >= rows || !live) return;
-  const int f = f0 + 4 * (lane >> 4);
-  float y[4] = {acc[0], acc[1], acc[2], acc[3]};
-  if (bias) {
-    const uint2 bv = *reinterpret_cast<const uint2*>(bias + f);
-    y[0] += bf16_bits_to_f32(bv.x & 0xffffu), y[1] += bf16_bits_to_f32(bv.x >> 16);
-    y[2] += bf16_bits_to_f32(bv.y & 0xffffu), y[3] += bf16_bits_to_f32(bv.y >> 16);
-  }
-  const uint2 o = {f32_to_bf16_bits(y[0]) | (f32_to_bf16_bits(y[1]) << 16),
-                   f32_to_bf16_bits(y[2]) | (f32_to_bf16_bits(y[3]) << 16)};
-  *reinterpret_cast<uint2*>(out + (int64_t)m * out_stride + f) = o;
 }
 
-template <int U, int KS>
-void launch_skinny(const void* x, int64_t xs, int64_t rows, int64_t k, const void* w, int64_t ws, int64_t n,
-                   const void* bias, void* out, int64_t os, hipStream_t st) {
-  const int64_t tiles = n / 16;
-  constexpr int kTiles = kWaves / KS;
-  hipLaunchKernelGGL((linear_skinny_kernel<U, KS>), dim3((unsigned)((tiles + kTiles - 1) / kTiles)), dim3(kThreads),
-                     0, st, static_cast<const char*>(x), xs * 2, (int)rows, (int)(k / 32), (int)tiles,
-                     static_cast<const char*>(w), ws * 2, static_cast<const uint16_t*>(bias),
-                     static_cast<uint16_t*>(out), os);
+// Sum of the K splits in order, bias, one rounding: four features per lane.
+__global__ __launch_bounds__(256) void linear_reduce_kernel(const float* __restrict__ partial, int splits, int rows,
+                                                            int n, const uint16_t* __restrict__ bias,
+                                                            uint16_t* __restrict__ out, int64_t out_stride) {
+  const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= rows * n) return;
+  const int row = i / n, f = i - row * n;
+  f32x4 y = *reinterpret_cast<const f32x4*>(partial + i);
+  for (int s = 1; s < splits; ++s) y += *reinterpret_cast<const f32x4*>(partial + (int64_t)s * rows * n + i);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (bias) y[e] += bf16_bits_to_f32(bias[f + e]);
+    out[row * out_stride + f + e] = (uint16_t)f32_to_bf16_bits(y[e]);
+  }
+}
+
+template <int U, int KS, int Z, int TF, int RB, int W>
+void launch(Args a, int64_t in_features, int splits, hipStream_t st) {
+  constexpr int kTiles = W / KS;
+  a.tiles = a.out_features / (16 / Z * TF);
+  a.k_steps = (int)(in_features / (32 * Z));
+  hipLaunchKernelGGL((linear_skinny_kernel<U, KS, Z, TF, RB, W>),
+                     dim3((unsigned)((a.tiles + kTiles - 1) / kTiles), (unsigned)splits), dim3(64 * W), 0, st, a);
+}
+
+// K splits across workgroups: one workgroup a CU (18944 x 3584, 32 rows: 43.0 us with 2 splits,
+// 46.9 with 1 or 4; 11008 x 2048: 20.1 with 4, 26 with 1).
+int num_splits(int64_t out_features) {
+  const int64_t tiles = out_features / 32;
+  const int64_t s = (256 + tiles / 2) / tiles;
+  return (int)(s < 1 ? 1 : s > 8 ? 8 : s);
+}
+
+int check(const void* x, int64_t xs, int64_t rows, int64_t max_rows, int64_t k, const void* w, int64_t ws, int64_t n,
+          const void* bias, const void* out, int64_t os) {
+  if (rows < 0 || rows > max_rows || k <= 0 || n <= 0) return VLC_ERR_INVALID;
+  if (k % 32 != 0 || n % 16 != 0) return VLC_ERR_UNSUPPORTED;
+  if (xs < k || ws < k || os < n) return VLC_ERR_INVALID;
+  if (rows == 0) return VLC_OK;
+  if (!x || !w || !out) return VLC_ERR_INVALID;
+  if (!aligned16(x) || !aligned16(w) || (xs % 8) || (ws % 8) || (reinterpret_cast<uintptr_t>(out) & 7) || (os % 4) ||
+      (bias && (reinterpret_cast<uintptr_t>(bias) & 7)))
+    return VLC_ERR_UNSUPPORTED;
+  if (n / 16 >= ((int64_t)1 << 26)) return VLC_ERR_UNSUPPORTED;
+  return VLC_OK;
 }
 
 }  // namespace
@@ -112,29 +185,73 @@ VLC_API int vlc_linear_skinny(const void* x, int64_t x_row_stride, int64_t rows,
                               const void* weight, int64_t w_row_stride, int64_t out_features, const void* bias,
                               void* out, int64_t out_row_stride, void* stream) {
   using namespace vlc;
-  if (rows < 0 || rows > kMaxRows || in_features <= 0 || out_features <= 0) return VLC_ERR_INVALID;
-  if (in_features % 32 != 0 || out_features % 16 != 0) return VLC_ERR_UNSUPPORTED;
-  if (x_row_stride < in_features || w_row_stride < in_features || out_row_stride < out_features)
-    return VLC_ERR_INVALID;
-  if (rows == 0) return VLC_OK;
-  if (!x || !weight || !out) return VLC_ERR_INVALID;
-  if (!aligned16(x) || !aligned16(weight) || (x_row_stride % 8) || (w_row_stride % 8) ||
-      (reinterpret_cast<uintptr_t>(out) & 7) || (out_row_stride % 4) || (bias && (reinterpret_cast<uintptr_t>(bias) & 7)))
-    return VLC_ERR_UNSUPPORTED;
-  if (out_features / 16 >= ((int64_t)1 << 30)) return VLC_ERR_UNSUPPORTED;
-  // Measured on the decode projections of Qwen2.5-VL-7B with cold weights (batch 4):
-  // 4 steps in flight per wave (U) beat 8 and 16 on every shape (fewer registers, more
-  // resident waves); a 4-way K split (two tiles per workgroup) was fastest from 288
-  // tiles up (QKV 11.8, gate/up 56.8, LM head 208.8 us) and an 8-way split for 224
-  // tiles (output projection 8.1, down projection 29.8 us), against 12.4, 56.7, 235.6,
-  // 12.1 and 48.2 us for the library GEMMs.
-  const int64_t tiles = out_features / 16;
+  const int bad = check(x, x_row_stride, rows, kMaxRows, in_features, weight, w_row_stride, out_features, bias, out,
+                        out_row_stride);
+  if (bad != VLC_OK || rows == 0) return bad;
+  const Args a = {static_cast<const char*>(x), x_row_stride * 2, (int)rows, 0, 0, static_cast<const char*>(weight),
+                  w_row_stride * 2, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(out), out_row_stride,
+                  nullptr, (int)out_features};
   hipStream_t st = as_stream(stream);
-  if (tiles <= 256)
-    launch_skinny<4, 8>(x, x_row_stride, rows, in_features, weight, w_row_stride, out_features, bias, out,
-                        out_row_stride, st);
+  const int64_t k = in_features, n = out_features;
+  // Z as large as the rows leave diagonal blocks free (and K divides); then as many tiles
+  // per x operand as leave about 200 workgroups (the figures at the head of the file).
+  if (rows <= 2 && k % 256 == 0)
+    launch<2, 4, 8, 1, 1, 4>(a, k, 1, st);
+  else if (rows <= 4 && k % 128 == 0) {
+    if (n >= 16 * 200)
+      launch<2, 8, 4, 4, 1, 8>(a, k, 1, st);
+    else
+      launch<2, 8, 4, 2, 1, 8>(a, k, 1, st);
+  } else if (rows <= 8 && k % 64 == 0) {
+    if (n >= 32 * 400 && n % 32 == 0)
+      launch<2, 4, 2, 4, 1, 4>(a, k, 1, st);
+    else if (n >= 16 * 200)
+      launch<2, 8, 2, 2, 1, 8>(a, k, 1, st);
+    else
+      launch<2, 8, 2, 1, 1, 8>(a, k, 1, st);
+  } else if (n >= 32 * 140 && n % 32 == 0 && k % 64 == 0) {
+    launch<2, 4, 2, 4, 2, 4>(a, k, 1, st);
+  } else {
+    launch<2, 8, 1, 1, 1, 8>(a, k, 1, st);
+  }
+  return launch_status();
+}
+
+VLC_API int64_t vlc_linear_split_workspace(int64_t rows, int64_t out_features) {
+  using namespace vlc;
+  if (rows <= 0 || rows > kMaxSplitRows || out_features < 32 || out_features >= ((int64_t)1 << 24)) return 0;
+  return num_splits(out_features) * rows * out_features * 4;
+}
+
+VLC_API int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
+                             const void* weight, int64_t w_row_stride, int64_t out_features, const void* bias,
+                             void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes,
+                             void* stream) {
+  using namespace vlc;
+  const int bad = check(x, x_row_stride, rows, kMaxSplitRows, in_features, weight, w_row_stride, out_features, bias,
+                        out, out_row_stride);
+  if (bad != VLC_OK || rows == 0) return bad;
+  if (out_features % 32 || out_features >= ((int64_t)1 << 24)) return VLC_ERR_UNSUPPORTED;
+  const int splits = num_splits(out_features);
+  if (splits > 1 && (!workspace || !aligned16(workspace) ||
+                     workspace_bytes < vlc_linear_split_workspace(rows, out_features)))
+    return VLC_ERR_WORKSPACE;
+  const Args a = {static_cast<const char*>(x), x_row_stride * 2, (int)rows, 0, 0, static_cast<const char*>(weight),
+                  w_row_stride * 2, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(out), out_row_stride,
+                  static_cast<float*>(workspace), (int)out_features};
+  hipStream_t st = as_stream(stream);
+  if (rows <= 16)
+    launch<2, 4, 1, 2, 1, 4>(a, in_features, splits, st);
+  else if (rows <= 32)
+    launch<2, 4, 1, 2, 2, 4>(a, in_features, splits, st);
+  else if (rows <= 48)
+    launch<2, 4, 1, 2, 3, 4>(a, in_features, splits, st);
   else
-    launch_skinny<4, 4>(x, x_row_stride, rows, in_features, weight, w_row_stride, out_features, bias, out,
-                        out_row_stride, st);
+    launch<2, 4, 1, 2, 4, 4>(a, in_features, splits, st);
+  const int st1 = launch_status();
+  if (st1 != VLC_OK || splits == 1) return st1;
+  const int64_t lanes = rows * out_features / 4;
+  hipLaunchKernelGGL(linear_reduce_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, st, a.partial, splits,
+                     (int)rows, (int)out_features, a.bias, a.out, out_row_stride);
   return launch_status();
 }

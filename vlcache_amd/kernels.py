@@ -673,16 +673,21 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
 
 
 # --------------------------------------------------------------------------- skinny linear
-SKINNY_MAX_ROWS = 16
+SKINNY_MAX_ROWS = 16  # vlc_linear_skinny
+SPLIT_MAX_ROWS = 64   # vlc_linear_split
 
 
 def linear_skinny_supported(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
     """Whether vlc_linear_skinny takes this call (bf16, at most 16 rows, K % 32, N % 16, aligned rows)."""
+    return _few_rows_supported(x, weight, bias, SKINNY_MAX_ROWS)
+
+
+def _few_rows_supported(x, weight, bias, max_rows: int) -> bool:
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2):
         return False
     m, k = x.shape
     n = weight.shape[0]
-    if m > SKINNY_MAX_ROWS or k % 32 or n % 16 or weight.shape[1] != k:
+    if m > max_rows or k % 32 or n % 16 or weight.shape[1] != k:
         return False
     if x.stride(1) != 1 or weight.stride(1) != 1 or x.stride(0) % 8 or weight.stride(0) % 8:
         return False
@@ -708,4 +713,27 @@ def linear_skinny(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
                                        bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
                                        _stream(x))
     _lib.check("vlc_linear_skinny", st)
+    return out
+
+
+def linear_split_supported(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
+    """Whether vlc_linear_split takes this call (as linear_skinny_supported, at most 64 rows, N % 32)."""
+    return _few_rows_supported(x, weight, bias, SPLIT_MAX_ROWS) and weight.shape[0] % 32 == 0
+
+
+def linear_split(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """x [M <= 64, K] @ weight[N, K]^T + bias with K split across workgroups (vlc_linear_split);
+    fp32 partial sums, one rounding to bf16."""
+    _require_device("linear_split", x, weight, bias)
+    if not linear_split_supported(x, weight, bias):
+        raise ValueError(f"linear_split does not take x {tuple(x.shape)} / weight {tuple(weight.shape)}")
+    m, k = x.shape
+    n = weight.shape[0]
+    lib = _lib.load()
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=x.device)
+    ws = torch.empty(lib.vlc_linear_split_workspace(m, n), dtype=torch.uint8, device=x.device)
+    st = lib.vlc_linear_split(x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0), n,
+                              bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
+                              ws.data_ptr(), ws.numel(), _stream(x))
+    _lib.check("vlc_linear_split", st)
     return out
