@@ -61,7 +61,7 @@ SIGNATURES = {
     "vlc_varlen_attn_fwd": (
         i32,
         [vp, i64, vp, i64, vp, i64, vp, i64, i32, i64, vp, vp, i32, i32, i32, i32, f32, i32,
-         c_i32p, vp, i64, vp, i64, vp, i64, vp],
+         vp, vp, i64, vp, i64, vp, i64, vp],
     ),
 }
 

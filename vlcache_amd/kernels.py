@@ -19,15 +19,17 @@ _PLAN_HEAD_DIM = 10  # header word of a vlc_attn_plan plan holding its head_dim
 ATTN_HEAD_DIMS = (128, 80)  # head_dims of vlc_varlen_attn_fwd (80: contiguous k/v only)
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# Host time per call bounds the short calls: a 160-token attention layer's three launches take
+# about 13 us of GPU time, and the two wrappers took 23 us of Python around them (now 12).  The
+# wrappers of the prefill path therefore read each tensor's shape and strides once, in tuples.
+def _stream(t: torch.Tensor) -> int:
+    """The current stream of t's device as a raw handle (0.1 us; a torch.cuda.Stream object costs 2)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _require_device(name: str, *tensors: torch.Tensor) -> None:
     for t in tensors:
-        if t is None:
-            continue
-        if not t.is_cuda:
+        if t is not None and not t.is_cuda:
             raise RuntimeError(f"{name}: tensors must be on a HIP device (got {t.device}); "
                                "the gfx950 kernels have no CPU path")
 
@@ -69,13 +71,22 @@ def store_kvcache_raw(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Ten
 
 
 # --------------------------------------------------------------------------- fused RoPE + scatter
-def _check_heads(name: str, t: torch.Tensor, n: int, heads: int, hd: int) -> None:
+def _check_heads(name: str, t: torch.Tensor, n: int, heads: int, hd: int) -> int:
+    """Checks a [n, heads, hd] tensor of contiguous head rows; returns its token stride."""
     if t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bf16")
-    if t.dim() != 3 or tuple(t.shape) != (n, heads, hd):
+    if t.shape != (n, heads, hd):
         raise ValueError(f"{name}: expected [{n}, {heads}, {hd}], got {tuple(t.shape)}")
-    if t.stride(-1) != 1 or t.stride(1) != hd:
+    st = t.stride()
+    if st[2] != 1 or st[1] != hd:
         raise ValueError(f"{name}: heads must be contiguous rows of {hd} elements")
+    return st[0]
+
+
+@functools.lru_cache(maxsize=64)
+def _section_array(section: tuple):
+    """The C array of an M-RoPE section triple (read by the host side of a call only)."""
+    return (ctypes.c_int32 * 3)(*section)
 
 
 def rope_store_kvcache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None,
@@ -98,30 +109,35 @@ def rope_store_kvcache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor
                     q_out, k_out)
     n, hq, hd = q.shape
     hkv = k.shape[1]
-    _check_heads("q", q, n, hq, hd)
-    _check_heads("k", k, n, hkv, hd)
-    if positions.dtype != torch.int64 or positions.stride(-1) != 1:
+    q_rs = _check_heads("q", q, n, hq, hd)
+    k_rs = _check_heads("k", k, n, hkv, hd)
+    pos_shape, pos_st = positions.shape, positions.stride()
+    if positions.dtype != torch.int64 or pos_st[-1] != 1:
         raise TypeError("positions must be int64 with contiguous rows")
-    if positions.dim() == 1:
+    if len(pos_shape) == 1:
         rows, pos_rs, sec = 1, 0, None
-        if positions.numel() != n:
+        if pos_shape[0] != n:
             raise ValueError("positions must hold one entry per token")
-    elif positions.dim() == 2 and positions.shape[0] == 3:
+    elif len(pos_shape) == 2 and pos_shape[0] == 3:
         if mrope_section is None:
             raise ValueError("[3, N] positions need mrope_section")
-        if positions.shape[1] != n:
+        if pos_shape[1] != n:
             raise ValueError("positions must hold one column per token")
-        rows, pos_rs = 3, positions.stride(0)
-        sec = (ctypes.c_int32 * 3)(*[int(x) for x in mrope_section])
+        rows, pos_rs = 3, pos_st[0]
+        sec = _section_array(tuple(int(x) for x in mrope_section))
     else:
         raise ValueError("positions must be [N] or [3, N]")
-    cs = cos_sin_cache
-    if cs.dtype != torch.float32 or cs.shape[-1] != hd or cs.stride(-1) != 1:
+    cs_shape, cs_st = cos_sin_cache.shape, cos_sin_cache.stride()
+    if cos_sin_cache.dtype != torch.float32 or cs_shape[-1] != hd or cs_st[-1] != 1:
         raise ValueError(f"cos_sin_cache must be fp32 [max_pos, (1,) {hd}] with contiguous rows")
-    if cs.dim() == 3 and cs.shape[1] != 1 or cs.dim() not in (2, 3):
+    if len(cs_shape) == 3 and cs_shape[1] != 1 or len(cs_shape) not in (2, 3):
         raise ValueError("cos_sin_cache must be [max_pos, hd] or [max_pos, 1, hd]")
     store = k_cache is not None or v_cache is not None
     num_slots = 0
+    kc_ptr = vc_ptr = slots_ptr = v_ptr = None
+    v_rs = 0
+    if v is not None:
+        v_ptr, v_rs = v.data_ptr(), v.stride(0)
     if store:
         if k_cache is None or v_cache is None or slot_mapping is None or v is None:
             raise ValueError("storing needs k_cache, v_cache, slot_mapping and v")
@@ -133,26 +149,27 @@ def rope_store_kvcache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor
         if k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16:
             raise TypeError("caches must be bf16")
         num_slots = k_cache.numel() // (hkv * hd)
-        if v_cache.numel() // (hkv * hd) != num_slots or k_cache.shape[-1] != hd or k_cache.shape[-2] != hkv:
+        kc_shape = k_cache.shape
+        if v_cache.numel() // (hkv * hd) != num_slots or kc_shape[-1] != hd or kc_shape[-2] != hkv:
             raise ValueError("caches must be [..., Hkv, hd] of equal size")
+        kc_ptr, vc_ptr, slots_ptr = k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr()
     if q_out is None:
-        q_out = torch.empty(n, hq, hd, dtype=torch.bfloat16, device=q.device)
+        q_out, qo_rs = torch.empty((n, hq, hd), dtype=torch.bfloat16, device=q.device), hq * hd
     else:
-        _check_heads("q_out", q_out, n, hq, hd)
+        qo_rs = _check_heads("q_out", q_out, n, hq, hd)
+    ko_ptr, ko_rs = None, 0
     if k_out is None and return_k:
-        k_out = torch.empty(n, hkv, hd, dtype=torch.bfloat16, device=q.device)
+        k_out = torch.empty((n, hkv, hd), dtype=torch.bfloat16, device=q.device)
+        ko_ptr, ko_rs = k_out.data_ptr(), hkv * hd
     elif k_out is not None:
-        _check_heads("k_out", k_out, n, hkv, hd)
+        ko_rs = _check_heads("k_out", k_out, n, hkv, hd)
+        ko_ptr = k_out.data_ptr()
     st = _lib.load().vlc_rope_store_kvcache(
-        q.data_ptr(), q.stride(0), q_out.data_ptr(), q_out.stride(0),
-        k.data_ptr(), k.stride(0), k_out.data_ptr() if k_out is not None else None,
-        k_out.stride(0) if k_out is not None else 0,
-        v.data_ptr() if v is not None else None, v.stride(0) if v is not None else 0,
-        hq, hkv, hd, positions.data_ptr(), rows, pos_rs, sec,
-        cs.data_ptr(), cs.stride(0), cs.shape[0],
-        k_cache.data_ptr() if store else None, v_cache.data_ptr() if store else None, num_slots,
-        slot_mapping.data_ptr() if store else None, n, _stream(q))
-    _lib.check("vlc_rope_store_kvcache", st)
+        q.data_ptr(), q_rs, q_out.data_ptr(), qo_rs, k.data_ptr(), k_rs, ko_ptr, ko_rs, v_ptr, v_rs,
+        hq, hkv, hd, positions.data_ptr(), rows, pos_rs, sec, cos_sin_cache.data_ptr(), cs_st[0], cs_shape[0],
+        kc_ptr, vc_ptr, num_slots, slots_ptr, n, _stream(q))
+    if st:
+        _lib.check("vlc_rope_store_kvcache", st)
     return q_out, k_out
 
 
@@ -245,6 +262,10 @@ class AttnPlan:
     cu_seqlens_q: tuple
     cu_seqlens_k: tuple
 
+    @functools.cached_property
+    def max_seqlen_k(self) -> int:
+        return max((b - a for a, b in zip(self.cu_seqlens_k, self.cu_seqlens_k[1:])), default=0)
+
     @property
     def num_items(self) -> int:
         return int(self.host[1])
@@ -309,13 +330,16 @@ def plan_attention(cu_seqlens_q, cu_seqlens_k, num_heads_q: int, num_heads_kv: i
                                list(np.asarray(cu_seqlens_k).tolist()), num_heads_q, num_heads_kv, causal)
 
 
-def _check_rows(name: str, t: torch.Tensor, heads: int) -> None:
+def _check_rows(name: str, t: torch.Tensor, heads: int):
+    """Checks [..., heads, 128] rows; returns the tensor's strides."""
     if t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bf16")
-    if t.shape[-1] != HEAD_DIM or t.shape[-2] != heads:
+    if t.shape[-2:] != (heads, HEAD_DIM):
         raise ValueError(f"{name}: expected [..., {heads}, {HEAD_DIM}], got {tuple(t.shape)}")
-    if t.stride(-1) != 1 or t.stride(-2) != HEAD_DIM:
+    st = t.stride()
+    if st[-1] != 1 or st[-2] != HEAD_DIM:
         raise ValueError(f"{name}: heads must be contiguous rows of {HEAD_DIM} elements")
+    return st
 
 
 def varlen_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -334,29 +358,30 @@ def varlen_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     0..95 of v (pass v zero-padded); output dims 96..127 are zero.
     """
     _require_device("varlen_attention", q, k, v, cu_seqlens_q, cu_seqlens_k, block_table)
-    hq = q.shape[1]
-    paged = block_table is not None
-    hkv = k.shape[-2]
-    _check_rows("q", q, hq)
-    _check_rows("k", k, hkv)
-    _check_rows("v", v, hkv)
+    q_shape, k_shape = q.shape, k.shape
+    hq, hkv = q_shape[1], k_shape[-2]
+    q_st = _check_rows("q", q, hq)
+    k_st = _check_rows("k", k, hkv)
+    v_st = _check_rows("v", v, hkv)
     if cu_seqlens_q.dtype != torch.int32 or cu_seqlens_k.dtype != torch.int32:
         raise TypeError("cu_seqlens must be int32")
     num_seqs = cu_seqlens_q.numel() - 1
+    paged = block_table is not None
     if paged:
-        if k.dim() != 4 or v.shape != k.shape:
+        bt_shape, bt_st = block_table.shape, block_table.stride()
+        if len(k_shape) != 4 or v.shape != k_shape:
             raise ValueError("paged k/v must be caches [num_blocks, page, Hkv, hd]")
-        if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.shape[0] != num_seqs:
+        if block_table.dtype != torch.int32 or len(bt_shape) != 2 or bt_shape[0] != num_seqs:
             raise ValueError("block_table must be int32 [num_seqs, max_blocks]")
-        if block_table.stride(1) != 1:
+        if bt_st[1] != 1:
             raise ValueError("block_table rows must be contiguous")
-        k_rs, v_rs = k.stride(1), v.stride(1)
-        if k.stride(0) != k.shape[1] * k_rs or v.stride(0) != v.shape[1] * v_rs:
+        nblocks, page = k_shape[0], k_shape[1]
+        k_rs, v_rs = k_st[1], v_st[1]
+        if k_st[0] != page * k_rs or v_st[0] != page * v_rs:
             raise ValueError("paged caches must have contiguous pages")
-        page, nblocks = k.shape[1], k.shape[0]
-        bt_ptr, bt_rs = block_table.data_ptr(), block_table.stride(0)
+        bt_ptr, bt_rs = block_table.data_ptr(), bt_st[0]
     else:
-        k_rs, v_rs = k.stride(0), v.stride(0)
+        k_rs, v_rs = k_st[0], v_st[0]
         page, nblocks, bt_ptr, bt_rs = 0, 0, None, 0
     if head_dim not in ATTN_HEAD_DIMS or (head_dim != HEAD_DIM and paged):
         raise ValueError(f"head_dim {head_dim} is not supported (128, or 80 with contiguous k/v)")
@@ -365,29 +390,30 @@ def varlen_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                               q.device)
     if plan.num_seqs != num_seqs or plan.num_heads_q != hq or plan.num_heads_kv != hkv or plan.causal != bool(causal):
         raise ValueError("attention plan does not match the call")
-    if int(plan.host[_PLAN_HEAD_DIM]) != head_dim:
-        raise ValueError(f"attention plan was built for head_dim {int(plan.host[_PLAN_HEAD_DIM])}, the call has {head_dim}")
+    host = plan.host
+    if host[_PLAN_HEAD_DIM] != head_dim:
+        raise ValueError(f"attention plan was built for head_dim {int(host[_PLAN_HEAD_DIM])}, the call has {head_dim}")
     # Bounds the kernel relies on, checked against the plan's host boundaries
     # (the device cu_seqlens must hold the same values).
-    if plan.cu_seqlens_q[-1] > q.shape[0]:
+    if plan.cu_seqlens_q[-1] > q_shape[0]:
         raise ValueError("cu_seqlens_q exceeds the rows of q")
     if paged:
-        max_sk = max((plan.cu_seqlens_k[i + 1] - plan.cu_seqlens_k[i] for i in range(num_seqs)), default=0)
-        if -(-max_sk // page) > block_table.shape[1]:
+        if -(-plan.max_seqlen_k // page) > bt_shape[1]:
             raise ValueError("block_table has fewer columns than the longest sequence needs")
-    elif plan.cu_seqlens_k[-1] > k.shape[0] or plan.cu_seqlens_k[-1] > v.shape[0]:
+    elif plan.cu_seqlens_k[-1] > k_shape[0] or plan.cu_seqlens_k[-1] > v.shape[0]:
         raise ValueError("cu_seqlens_k exceeds the rows of k/v")
     if out is None:
-        out = torch.empty(q.shape[0], hq, HEAD_DIM, dtype=torch.bfloat16, device=q.device)
+        out = torch.empty((q_shape[0], hq, HEAD_DIM), dtype=torch.bfloat16, device=q.device)
     ws = plan.workspace
     st = _lib.load().vlc_varlen_attn_fwd(
-        q.data_ptr(), q.stride(0), k.data_ptr(), k_rs, v.data_ptr(), v_rs,
+        q.data_ptr(), q_st[0], k.data_ptr(), k_rs, v.data_ptr(), v_rs,
         bt_ptr, bt_rs, page, nblocks, cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
         num_seqs, hq, hkv, head_dim, float(softmax_scale), 1 if causal else 0,
-        plan.host.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), plan.dev.data_ptr(), plan.host.size,
+        host.__array_interface__["data"][0], plan.dev.data_ptr(), host.size,
         out.data_ptr(), out.stride(0), ws.data_ptr() if ws is not None else None,
         ws.numel() if ws is not None else 0, _stream(q))
-    _lib.check("vlc_varlen_attn_fwd", st)
+    if st:
+        _lib.check("vlc_varlen_attn_fwd", st)
     return out
 
 
