@@ -353,6 +353,21 @@ int vlc_silu_mul(const void* gate_up, int64_t gate_up_row_stride, int64_t num_ro
                  void* out, int64_t out_row_stride, void* stream);
 
 /*
+ * The same with columns inter .. out_width - 1 of out written as zero (out_width % 4 == 0,
+ * out_row_stride >= out_width): the input of a product over a padded K.
+ */
+int vlc_silu_mul_padded(const void* gate_up, int64_t gate_up_row_stride, int64_t num_rows, int64_t inter,
+                        void* out, int64_t out_row_stride, int64_t out_width, void* stream);
+
+/*
+ * dst[r][c] = src[r][c] for c < cols, 0 for cols <= c < width (16-bit elements): a weight's
+ * rows padded to an aligned length.  cols % 4 == 0, width % 8 == 0; src 8-byte aligned with a
+ * row stride multiple of 4 elements, dst 16-byte aligned with a row stride multiple of 8.
+ */
+int vlc_pad_rows(const void* src, int64_t src_row_stride, int64_t num_rows, int64_t cols,
+                 void* dst, int64_t dst_row_stride, int64_t width, void* stream);
+
+/*
  * Skinny linear layer (M <= 16 rows): out[m][n] = bf16(sum_k x[m][k] * weight[n][k] + bias[n]),
  * fp32 accumulation.  Replaces the decode-step projections of the decoder
  * (QKVParallelLinear / RowParallelLinear / MergedColumnParallelLinear and the LM head,

@@ -220,3 +220,32 @@ def test_linear_split(dev, m, k, n, bias):
                 lin.bias.copy_(bd)
             assert torch.equal(lin(xd), out)
         assert lin(xd).requires_grad  # with gradients on, the layer stays torch's
+
+
+@pytest.mark.parametrize("rows,inter,width", [(1, 4, 8), (5, 3420, 3456), (1300, 3420, 3456), (1300, 3416, 3416),
+                                              (700, 2044, 2048)])
+def test_silu_mul_padded(dev, rows, inter, width):
+    """Both access widths, a last 16-byte group that is half past inter, gate/up rows with a gap and
+    without one (the last row ends the buffer): the same bits as the unpadded kernel's oracle bar, zero tail."""
+    from vlcache_amd import kernels
+
+    say(f"silu_mul_padded rows={rows} inter={inter} width={width}")
+    gu = randn_bf16((rows, 2 * inter), rows + inter, 3.0)
+    wide = torch.full((rows, 2 * inter + 8), float("nan"), dtype=torch.bfloat16, device=dev)
+    wide[:, :-8] = gu.to(dev)
+    for src in (gu.to(dev), wide[:, :-8]):
+        out = kernels.silu_mul_padded(src, width)
+        _within_ulps(out[:, :inter].contiguous(), ol.silu_mul(gu), f"silu_mul_padded {rows}x{inter}")
+        assert not out[:, inter:].view(torch.int16).any()
+
+
+@pytest.mark.parametrize("rows,cols,width", [(1, 4, 8), (1280, 3420, 3456), (33, 3416, 3416), (7, 100, 256)])
+def test_pad_rows(dev, rows, cols, width):
+    from vlcache_amd import kernels
+
+    say(f"pad_rows {rows}x{cols} -> {width}")
+    x = randn_bf16((rows, cols + 4), rows)
+    for src in (x[:, :cols].contiguous(), x[:, :cols]):
+        out = kernels.pad_rows(src.to(dev) if src.is_contiguous() else x.to(dev)[:, :cols], width).cpu()
+        assert torch.equal(out[:, :cols].view(torch.int16), src.contiguous().view(torch.int16))
+        assert not out[:, cols:].view(torch.int16).any()

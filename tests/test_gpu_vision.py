@@ -338,3 +338,41 @@ def test_window_attention_refuses_long_windows_and_bad_boundaries(dev):
         cu = np.asarray(bad, dtype=np.int32)
         with pytest.raises(RuntimeError, match=f"status {status}"):
             kernels.vision_window_attention(qkv.to(dev), pos, cos, sin, cu, torch.from_numpy(cu).to(dev), 16, 0.1)
+
+
+@pytest.mark.parametrize("rows", [5, 1023, 1024, 1500])
+def test_vision_mlp_padded_products(dev, rows):
+    """VisionMLP at the published widths on both sides of its padding rule against the fp32 oracle of
+    its parts, with its own parameters, after an in-place update of them, and with parameters copied
+    without the spare rows (which run the plain product); bar: bf16 rounding of the 3420-wide hidden
+    row and of the result, 2^-7 of the row's norm."""
+    import copy
+
+    from oracle import layers as ol
+    from vlcache_amd.vision import VisionMLP
+
+    say(f"vision MLP rows={rows}")
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(dev):
+            mlp = VisionMLP(1280, 3420)
+    finally:
+        torch.set_default_dtype(prev)
+    x = torch.randn(rows, 1280, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16)
+
+    def check(m, what):
+        with torch.inference_mode():
+            got = m(x.to(dev)).float().cpu()
+        g, d = m.gate_up_proj, m.down_proj
+        gu = (x.float() @ g.weight.float().cpu().t() + g.bias.float().cpu()).to(torch.bfloat16)
+        ref = ol.silu_mul(gu).float() @ d.weight.float().cpu().t() + d.bias.float().cpu()
+        assert ((got - ref).norm(dim=1) <= 2.0 ** -7 * ref.norm(dim=1)).all(), what
+
+    assert mlp.gate_up_proj.weight.shape == (6840, 1280) and mlp.gate_up_proj.weight.is_contiguous()
+    check(mlp, "as built")
+    with torch.no_grad():
+        mlp.down_proj.weight.data.mul_(-0.5)
+        mlp.gate_up_proj.weight.data.mul_(2)
+    check(mlp, "after an update in place")
+    check(copy.deepcopy(mlp), "copied")

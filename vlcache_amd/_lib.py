@@ -51,6 +51,8 @@ SIGNATURES = {
     "vlc_vision_window_attn": (i32, [vp, i64, vp, vp, vp, i64, vp, vp, i32, i64, i32, i32, f32, vp, i64, vp]),
     "vlc_rms_norm": (i32, [vp, i64, vp, i64, vp, i64, vp, f32, i64, i64, vp, i64, vp]),
     "vlc_silu_mul": (i32, [vp, i64, i64, i64, vp, i64, vp]),
+    "vlc_silu_mul_padded": (i32, [vp, i64, i64, i64, vp, i64, i64, vp]),
+    "vlc_pad_rows": (i32, [vp, i64, i64, i64, vp, i64, i64, vp]),
     "vlc_linear_skinny": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, vp]),
     "vlc_linear_split_workspace": (i64, [i64, i64]),
     "vlc_linear_split": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, vp, i64, vp]),

@@ -13,7 +13,7 @@
 //
 // silu_mul follows layers/activation.py:8-14 (SiluAndMul: chunk the last dim
 // into gate and up, silu(gate) * up) with fp32 math and one rounding to bf16,
-// as the reference's compiled kernel computes it.  A lane owns 4 elements.
+// as the reference's compiled kernel computes it.
 #include "common.h"
 
 namespace vlc {
@@ -123,25 +123,30 @@ int launch_rms(const void* x, int64_t xs, const void* res, int64_t rs, void* ro,
   return launch_status();
 }
 
-// V = 8: 16-byte accesses (inter % 8 == 0), else 8-byte ones (V = 4).
-template <int V>
+// A lane owns V elements of a row (V = 8: 16-byte accesses of gate and out; the up half
+// starts at any multiple of 8 bytes).  Columns inter .. width - 1 of out are written as
+// zero; a lane whose last four elements lie past inter loads only the first four.  Bound by
+// memory: 42196 x 3420 reads and writes 866 MB.
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+template <int V, typename Index>
 __global__ __launch_bounds__(kThreads) void silu_mul_kernel(const char* __restrict__ gu, int64_t gu_stride_b,
-                                                            int64_t rows, int groups, int64_t up_offset_b,
+                                                            Index rows, Index groups, int inter,
                                                             char* __restrict__ out, int64_t out_stride_b) {
-  const int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const Index u = (Index)blockIdx.x * kThreads + threadIdx.x;
   if (u >= rows * groups) return;
-  const int64_t row = u / groups;
-  const int q = (int)(u - row * groups);
-  const char* src = gu + row * gu_stride_b + (int64_t)q * (2 * V);
-  uint32_t g[V / 2], p[V / 2];
-  if constexpr (V == 8) {
+  const Index row = u / groups;
+  const int c = (int)(u - row * groups) * V;
+  const char* src = gu + row * gu_stride_b + (int64_t)c * 2;
+  const char* up = src + (int64_t)inter * 2;
+  uint32_t g[V / 2] = {}, p[V / 2] = {};
+  if (V == 8 && c + 8 <= inter) {
     const u32x4 a = *reinterpret_cast<const u32x4*>(src);
-    const u32x4 b = *reinterpret_cast<const u32x4*>(src + up_offset_b);
-    g[0] = a.x, g[1] = a.y, g[2] = a.z, g[3] = a.w;
-    p[0] = b.x, p[1] = b.y, p[2] = b.z, p[3] = b.w;
-  } else {
+    const u32x4_a8 b = *reinterpret_cast<const u32x4_a8*>(up);
+    g[0] = a.x, g[1] = a.y, g[V / 2 - 2] = a.z, g[V / 2 - 1] = a.w;
+    p[0] = b[0], p[1] = b[1], p[V / 2 - 2] = b[2], p[V / 2 - 1] = b[3];
+  } else if (c < inter) {
     const uint2 a = *reinterpret_cast<const uint2*>(src);
-    const uint2 b = *reinterpret_cast<const uint2*>(src + up_offset_b);
+    const uint2 b = *reinterpret_cast<const uint2*>(up);
     g[0] = a.x, g[1] = a.y;
     p[0] = b.x, p[1] = b.y;
   }
@@ -151,11 +156,34 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(const char* __restri
     const float g0 = lo16(g[k]), g1 = hi16(g[k]);
     o[k] = pack2(g0 / (1.0f + expf(-g0)) * lo16(p[k]), g1 / (1.0f + expf(-g1)) * hi16(p[k]));
   }
-  char* dst = out + row * out_stride_b + (int64_t)q * (2 * V);
+  char* dst = out + row * out_stride_b + (int64_t)c * 2;
   if constexpr (V == 8)
     *reinterpret_cast<u32x4*>(dst) = u32x4{o[0], o[1], o[2], o[3]};
   else
     *reinterpret_cast<uint2*>(dst) = uint2{o[0], o[1]};
+}
+
+// dst[r][c] = src[r][c] for c < cols, 0 for cols <= c < width; a lane per 16-byte chunk of dst.
+__global__ __launch_bounds__(kThreads) void pad_rows_kernel(const char* __restrict__ src, int64_t src_stride_b,
+                                                            uint32_t chunks, uint32_t per_row, int cols,
+                                                            char* __restrict__ dst, int64_t dst_stride_b) {
+  const uint32_t u = blockIdx.x * kThreads + threadIdx.x;
+  if (u >= chunks) return;
+  const uint32_t row = u / per_row, c = (u - row * per_row) * 8;
+  const char* s = src + row * src_stride_b + (int64_t)c * 2;
+  uint2 a = {0u, 0u}, b = {0u, 0u};
+  if ((int)c < cols) a = *reinterpret_cast<const uint2*>(s);
+  if ((int)c + 4 < cols) b = *reinterpret_cast<const uint2*>(s + 8);
+  *reinterpret_cast<u32x4*>(dst + row * dst_stride_b + (int64_t)c * 2) = u32x4{a.x, a.y, b.x, b.y};
+}
+
+template <int V, typename Index>
+void launch_silu(const void* gate_up, int64_t gus, int64_t rows, int64_t inter, void* out, int64_t os, int64_t width,
+                 hipStream_t st) {
+  const int64_t groups = width / V, blocks = (rows * groups + kThreads - 1) / kThreads;
+  hipLaunchKernelGGL((silu_mul_kernel<V, Index>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
+                     static_cast<const char*>(gate_up), gus * 2, (Index)rows, (Index)groups, (int)inter,
+                     static_cast<char*>(out), os * 2);
 }
 
 }  // namespace
@@ -196,11 +224,13 @@ VLC_API int vlc_rms_norm(const void* x, int64_t x_row_stride, const void* residu
 #undef VLC_RMS_CASE
 }
 
-VLC_API int vlc_silu_mul(const void* gate_up, int64_t gate_up_row_stride, int64_t num_rows, int64_t inter,
-                         void* out, int64_t out_row_stride, void* stream) {
+VLC_API int vlc_silu_mul_padded(const void* gate_up, int64_t gate_up_row_stride, int64_t num_rows, int64_t inter,
+                                void* out, int64_t out_row_stride, int64_t out_width, void* stream) {
   using namespace vlc;
-  if (num_rows < 0 || inter <= 0 || inter % 4 != 0) return VLC_ERR_INVALID;
-  if (gate_up_row_stride < 2 * inter || out_row_stride < inter) return VLC_ERR_INVALID;
+  if (num_rows < 0 || inter <= 0 || inter % 4 != 0 || inter >= ((int64_t)1 << 30) || out_width < inter ||
+      out_width % 4 != 0)
+    return VLC_ERR_INVALID;
+  if (gate_up_row_stride < 2 * inter || out_row_stride < out_width) return VLC_ERR_INVALID;
   if (num_rows == 0) return VLC_OK;
   if (!gate_up || !out) return VLC_ERR_INVALID;
   if ((reinterpret_cast<uintptr_t>(gate_up) & 7) || (reinterpret_cast<uintptr_t>(out) & 7) ||
@@ -209,19 +239,43 @@ VLC_API int vlc_silu_mul(const void* gate_up, int64_t gate_up_row_stride, int64_
   // 16-byte accesses when the call is large enough to fill the device with half as
   // many lanes: 1247 x 11008 in 17.2 against 18.9 us, 10741 x 11008 in 125 against
   // 139 us; a decode step's 4 x 18944 measured 2.2 against 2.05 us with them.
-  const bool v16 = inter % 8 == 0 && num_rows * inter >= ((int64_t)1 << 20) && aligned16(gate_up) &&
+  const bool v16 = out_width % 8 == 0 && num_rows * inter >= ((int64_t)1 << 20) && aligned16(gate_up) &&
                    aligned16(out) && gate_up_row_stride % 8 == 0 && out_row_stride % 8 == 0;
-  const int groups = (int)(inter / (v16 ? 8 : 4));
-  const int64_t total = num_rows * groups;
-  const int64_t blocks = (total + kThreads - 1) / kThreads;
-  if (blocks >= ((int64_t)1 << 31)) return VLC_ERR_UNSUPPORTED;
-  if (v16)
-    hipLaunchKernelGGL(silu_mul_kernel<8>, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream),
-                       static_cast<const char*>(gate_up), gate_up_row_stride * 2, num_rows, groups, inter * 2,
-                       static_cast<char*>(out), out_row_stride * 2);
+  const int64_t total = num_rows * (out_width / (v16 ? 8 : 4));
+  if (total / kThreads >= ((int64_t)1 << 31) - 1) return VLC_ERR_UNSUPPORTED;
+  // 32-bit lane indices where they fit: a 64-bit division costs a lane as much as its exps
+  const bool small = total < ((int64_t)1 << 31);
+  hipStream_t st = as_stream(stream);
+  if (v16 && small)
+    launch_silu<8, uint32_t>(gate_up, gate_up_row_stride, num_rows, inter, out, out_row_stride, out_width, st);
+  else if (v16)
+    launch_silu<8, int64_t>(gate_up, gate_up_row_stride, num_rows, inter, out, out_row_stride, out_width, st);
+  else if (small)
+    launch_silu<4, uint32_t>(gate_up, gate_up_row_stride, num_rows, inter, out, out_row_stride, out_width, st);
   else
-    hipLaunchKernelGGL(silu_mul_kernel<4>, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream),
-                       static_cast<const char*>(gate_up), gate_up_row_stride * 2, num_rows, groups, inter * 2,
-                       static_cast<char*>(out), out_row_stride * 2);
+    launch_silu<4, int64_t>(gate_up, gate_up_row_stride, num_rows, inter, out, out_row_stride, out_width, st);
+  return launch_status();
+}
+
+VLC_API int vlc_silu_mul(const void* gate_up, int64_t gate_up_row_stride, int64_t num_rows, int64_t inter,
+                         void* out, int64_t out_row_stride, void* stream) {
+  return vlc_silu_mul_padded(gate_up, gate_up_row_stride, num_rows, inter, out, out_row_stride, inter, stream);
+}
+
+VLC_API int vlc_pad_rows(const void* src, int64_t src_row_stride, int64_t num_rows, int64_t cols, void* dst,
+                         int64_t dst_row_stride, int64_t width, void* stream) {
+  using namespace vlc;
+  if (num_rows < 0 || cols <= 0 || cols % 4 != 0 || width < cols || width % 8 != 0 || src_row_stride < cols ||
+      dst_row_stride < width)
+    return VLC_ERR_INVALID;
+  if (num_rows == 0) return VLC_OK;
+  if (!src || !dst) return VLC_ERR_INVALID;
+  if ((reinterpret_cast<uintptr_t>(src) & 7) || src_row_stride % 4 || !aligned16(dst) || dst_row_stride % 8)
+    return VLC_ERR_UNSUPPORTED;
+  const int64_t chunks = num_rows * (width / 8);
+  if (chunks >= ((int64_t)1 << 31) || width >= ((int64_t)1 << 30)) return VLC_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((chunks + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                     as_stream(stream), static_cast<const char*>(src), src_row_stride * 2, (uint32_t)chunks,
+                     (uint32_t)(width / 8), (int)cols, static_cast<char*>(dst), dst_row_stride * 2);
   return launch_status();
 }

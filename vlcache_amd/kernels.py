@@ -698,6 +698,32 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
     return o.view(*lead, inter)
 
 
+def silu_mul_padded(gate_up: torch.Tensor, width: int) -> torch.Tensor:
+    """silu_mul of [rows, 2 * inter] rows into [rows, width], columns inter .. width - 1 zero
+    (vlc_silu_mul_padded)."""
+    _require_device("silu_mul_padded", gate_up)
+    if gate_up.dim() != 2 or gate_up.shape[1] % 2:
+        raise ValueError("gate_up must be [rows, 2 * inter]")
+    rows, two = gate_up.shape
+    _rows2d("gate_up", gate_up, two)
+    out = torch.empty(rows, width, dtype=torch.bfloat16, device=gate_up.device)
+    st = _lib.load().vlc_silu_mul_padded(gate_up.data_ptr(), gate_up.stride(0), rows, two // 2, out.data_ptr(),
+                                         width, width, _stream(gate_up))
+    _lib.check("vlc_silu_mul_padded", st)
+    return out
+
+
+def pad_rows(x: torch.Tensor, width: int) -> torch.Tensor:
+    """A copy of x [rows, cols] bf16 with rows zero-padded to width (vlc_pad_rows)."""
+    _require_device("pad_rows", x)
+    rows, cols = x.shape
+    _rows2d("x", x, cols)
+    out = torch.empty(rows, width, dtype=torch.bfloat16, device=x.device)
+    st = _lib.load().vlc_pad_rows(x.data_ptr(), x.stride(0), rows, cols, out.data_ptr(), width, width, _stream(x))
+    _lib.check("vlc_pad_rows", st)
+    return out
+
+
 # --------------------------------------------------------------------------- skinny linear
 SKINNY_MAX_ROWS = 16  # vlc_linear_skinny
 SPLIT_MAX_ROWS = 64   # vlc_linear_split
