@@ -397,6 +397,21 @@ int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, int64_t 
                      void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes,
                      void* stream);
 
+/*
+ * Gate/up projection with SiLU-and-multiply, for many rows: out[m][i] = bf16(silu(gate) * up),
+ * gate = bf16(sum_k x[m][k] weight[i][k] + bias[i]), up the same with row inter + i; fp32
+ * accumulation.  MergedColumnParallelLinear and SiluAndMul (models/qwen3.py:112-127,
+ * layers/activation.py:8-14), and the vision MLP's (models/qwen2_5_vl.py:219-243), in one launch.
+ * weight: [2 * inter, in_features] bf16; bias: bf16 [2 * inter] or NULL; columns
+ * inter .. out_width - 1 of out are written as zero.  in_features % 64 == 0, inter % 4 == 0,
+ * out_width % 4 == 0 and at most inter rounded up to 128; x and weight 16-byte aligned with row
+ * strides multiples of 8 elements and below 2^22; out and bias 8-byte aligned, out_row_stride a
+ * multiple of 4 (VLC_ERR_UNSUPPORTED otherwise).
+ */
+int vlc_linear_silu(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
+                    const void* weight, int64_t w_row_stride, int64_t inter, const void* bias,
+                    void* out, int64_t out_row_stride, int64_t out_width, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -249,3 +249,72 @@ def test_pad_rows(dev, rows, cols, width):
         out = kernels.pad_rows(src.to(dev) if src.is_contiguous() else x.to(dev)[:, :cols], width).cpu()
         assert torch.equal(out[:, :cols].view(torch.int16), src.contiguous().view(torch.int16))
         assert not out[:, cols:].view(torch.int16).any()
+
+
+@pytest.mark.parametrize("m,k,inter,bias,width", [(1, 64, 4, True, None), (255, 128, 124, False, 128),
+                                                  (256, 192, 128, True, None), (257, 256, 132, True, 256),
+                                                  (700, 1280, 3420, True, 3456), (2100, 2048, 384, False, None)])
+def test_linear_silu(dev, m, k, inter, bias, width):
+    """vlc_linear_silu against the oracle's SiLU of the exact product's bf16 gate and up: one token and one
+    group of features, rows and features around the 256 x 128 tile, 1 to 32 K steps, a zero tail, rows with a
+    gap.  An fp32 sum next to a rounding boundary may round the other way (sums in another order): gate and
+    up are then each off by 2^-8 of themselves, silu' <= 1.1, and the result rounds once more, which is at most
+    2^-8 (1.1 + 1 + 0.5) |gate| |up| < 2^-6 (1 + |gate|) (1 + |up|) for all; 99 % are equal."""
+    from vlcache_amd import kernels
+
+    say(f"linear_silu m={m} k={k} inter={inter} bias={bias} width={width}")
+    wide = torch.full((m, k + 8), float("nan"), dtype=torch.bfloat16, device=dev)
+    x, w = randn_bf16((m, k), m + k), randn_bf16((2 * inter, k), k + inter, 0.05)
+    b = randn_bf16((2 * inter,), 5) if bias else None
+    wide[:, :-8] = x.to(dev)
+    gu = (x.double() @ w.double().t() + (b.double() if bias else 0.0)).float().to(torch.bfloat16)
+    ref = ol.silu_mul(gu).float()
+    scale = (1 + gu[:, :inter].float().abs()) * (1 + gu[:, inter:].float().abs())
+    for src in (x.to(dev), wide[:, :-8]):
+        full = kernels.linear_silu(src, w.to(dev), b.to(dev) if bias else None, width)
+        out = full[:, :inter].float().cpu()
+        assert ((out - ref).abs() <= 2.0 ** -6 * scale).all()
+        assert float((out == ref).float().mean()) >= 0.99 or out.numel() < 200
+        assert not full[:, inter:].view(torch.int16).any()
+
+
+def test_linear_silu_extremes(dev):
+    """Gates whose exponential overflows or vanishes, infinities and NaN: as SiLU-and-multiply itself."""
+    from vlcache_amd import kernels
+
+    say("linear_silu extremes")
+    gates = torch.tensor([-1e30, -100.0, -88.5, -20.0, -0.0, 0.0, 20.0, 100.0, 1e30, float("inf"), float("-inf"),
+                          float("nan")]).to(torch.bfloat16)
+    x = torch.zeros(12, 64, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = 1.0, torch.arange(12)
+    w = torch.zeros(2 * 12, 64, dtype=torch.bfloat16)
+    b = torch.cat([gates, torch.full((12,), 2.0)]).to(torch.bfloat16)
+    out = kernels.linear_silu(x.to(dev), w.to(dev), b.to(dev)).float().cpu()
+    ref = kernels.silu_mul(b[None].expand(12, -1).contiguous().to(dev)).float().cpu()
+    same = (out == ref) | (out.isnan() & ref.isnan()) | ((out - ref).abs() <= ref.abs() * 2.0 ** -7 + 1e-36)
+    assert same.all(), (out[0].tolist(), ref[0].tolist())
+
+
+@pytest.mark.parametrize("rows,inter,pays", [(1247, 11008, True), (1300, 11008, False), (511, 18944, False),
+                                             (1000, 18944, True)])
+def test_decoder_mlp_route(dev, rows, inter, pays):
+    """The decoder MLP on each side of the rule: the same values as its parts, and hooks are honoured."""
+    from types import SimpleNamespace
+
+    from vlcache_amd import kernels
+    from vlcache_amd.qwen_vl import MLP
+
+    say(f"decoder MLP route rows={rows} inter={inter}")
+    assert kernels.linear_silu_pays(rows, inter) is pays
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(dev):
+            mlp = MLP(SimpleNamespace(hidden_size=256, intermediate_size=inter))
+    finally:
+        torch.set_default_dtype(prev)
+    x = randn_bf16((rows, 256), rows).to(dev)
+    with torch.inference_mode():
+        got = mlp(x).float()
+        ref = mlp.down_proj(kernels.silu_mul(mlp.gate_up_proj(x))).float()
+    assert (got - ref).norm() <= 2.0 ** -8 * ref.norm()

@@ -340,12 +340,11 @@ def test_window_attention_refuses_long_windows_and_bad_boundaries(dev):
             kernels.vision_window_attention(qkv.to(dev), pos, cos, sin, cu, torch.from_numpy(cu).to(dev), 16, 0.1)
 
 
-@pytest.mark.parametrize("rows", [5, 1023, 1024, 1500])
-def test_vision_mlp_padded_products(dev, rows):
-    """VisionMLP at the published widths on both sides of its padding rule against the fp32 oracle of
-    its parts, with its own parameters, after an in-place update of them, and with parameters copied
-    without the spare rows (which run the plain product); bar: bf16 rounding of the 3420-wide hidden
-    row and of the result, 2^-7 of the row's norm."""
+@pytest.mark.parametrize("rows", [5, 1279, 1280, 1500])
+def test_vision_mlp_fused_products(dev, rows):
+    """VisionMLP at the published widths on both sides of its rule against the fp32 oracle of its parts,
+    as built, after an in-place update of its parameters, copied, and with a hook on its projections (which
+    then are called); bar: bf16 rounding of the 3420-wide hidden row and of the result, 2^-7 of the row's norm."""
     import copy
 
     from oracle import layers as ol
@@ -369,10 +368,14 @@ def test_vision_mlp_padded_products(dev, rows):
         ref = ol.silu_mul(gu).float() @ d.weight.float().cpu().t() + d.bias.float().cpu()
         assert ((got - ref).norm(dim=1) <= 2.0 ** -7 * ref.norm(dim=1)).all(), what
 
-    assert mlp.gate_up_proj.weight.shape == (6840, 1280) and mlp.gate_up_proj.weight.is_contiguous()
     check(mlp, "as built")
     with torch.no_grad():
         mlp.down_proj.weight.data.mul_(-0.5)
         mlp.gate_up_proj.weight.data.mul_(2)
     check(mlp, "after an update in place")
     check(copy.deepcopy(mlp), "copied")
+    calls = []
+    for part in (mlp.gate_up_proj, mlp.down_proj):
+        part.register_forward_hook(lambda *a: calls.append(1))
+    check(mlp, "hooked")
+    assert len(calls) == 2

@@ -789,3 +789,55 @@ def linear_split(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
                               ws.data_ptr(), ws.numel(), _stream(x))
     _lib.check("vlc_linear_split", st)
     return out
+
+
+# --------------------------------------------------------------------------- gate/up projection
+def linear_silu_supported(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
+    """Whether vlc_linear_silu takes this call (bf16, K % 64, whole groups of 4 features, aligned rows)."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2):
+        return False
+    k, n = x.shape[1], weight.shape[0]
+    xs, ws = x.stride(), weight.stride()
+    if weight.shape[1] != k or k % 64 or n % 8 or xs[1] != 1 or ws[1] != 1 or xs[0] % 8 or ws[0] % 8:
+        return False
+    if xs[0] < k or ws[0] < k or max(xs[0], ws[0]) >= 1 << 22 or x.data_ptr() % 16 or weight.data_ptr() % 16:
+        return False
+    return bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 8 == 0)
+
+
+def plain_linear(m: torch.nn.Module) -> bool:
+    """Whether calling m is no more than its product: an nn.Linear without hooks, whose call a fused kernel
+    may stand in for."""
+    return type(m).forward in _LINEAR_FORWARDS and not (m._forward_hooks or m._forward_pre_hooks)
+
+
+_LINEAR_FORWARDS = {torch.nn.Linear.forward}  # layers.linear.Linear adds its own
+
+
+def linear_silu_pays(rows: int, inter: int) -> bool:
+    """Whether vlc_linear_silu beats the library's product and the SiLU kernel on a tile-aligned inter: the
+    256 x 128 tiles run in rounds of one per CU, and 70 % or more of the rounds' tiles has to be work.  Library
+    / fused time at that share: 2048 -> 22016 0.57 0.90, 0.66 1.04, 0.69 0.96, 0.70 1.22, 0.82 1.10; 3584 -> 37888
+    0.72 1.09, 0.73 1.00, 0.75 1.29, 0.79 1.10, 0.94 1.42.  Below 512 rows the library was faster."""
+    tiles = -(-rows // 256) * -(-inter // 128)
+    return rows >= 512 and rows * inter >= 0.7 * (-(-tiles // 256) * 256) * (256 * 128)
+
+
+def linear_silu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
+                width: int | None = None) -> torch.Tensor:
+    """silu(gate) * up of x [M, K] @ weight [2 * inter, K]^T + bias (vlc_linear_silu) -> [M, width], columns
+    inter .. width - 1 zero (width: inter by default, at most inter rounded up to 128)."""
+    _require_device("linear_silu", x, weight, bias)
+    if not linear_silu_supported(x, weight, bias):
+        raise ValueError(f"linear_silu does not take x {tuple(x.shape)} / weight {tuple(weight.shape)}")
+    m, k = x.shape
+    inter = weight.shape[0] // 2
+    if bias is not None and bias.numel() != 2 * inter:
+        raise ValueError("bias must hold one entry per weight row")
+    width = inter if width is None else width
+    out = torch.empty((m, width), dtype=torch.bfloat16, device=x.device)
+    st = _lib.load().vlc_linear_silu(x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0), inter,
+                                     bias.data_ptr() if bias is not None else None, out.data_ptr(), width, width,
+                                     _stream(x))
+    _lib.check("vlc_linear_silu", st)
+    return out

@@ -10,7 +10,8 @@ GEMMs run on torch (hipBLASLt) except calls of at most 16 rows (decode steps),
 which stream the weights through vlc_linear_skinny (layers.linear.Linear); per layer the rotary
 embedding of q and k and the KV store run as one gfx950 kernel and the
 attention as another (layers.attention.Attention), each RMSNorm (with its
-residual add) as one kernel and the MLP's SiLU-and-multiply as one.
+residual add) as one kernel and the MLP's SiLU-and-multiply as one, or for many
+rows as the epilogue of its gate/up projection (vlc_linear_silu).
 When the model config carries a vision_config the model owns the vision tower
 (vision.VisionTransformer, the cold path behind the encoder cache).
 Weights are random N(0, 0.02) unless loaded by the caller.
@@ -74,7 +75,11 @@ class MLP(nn.Module):
         self.down_proj = Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, x):
-        return self.down_proj(kernels.silu_mul(self.gate_up_proj(x)))
+        g = self.gate_up_proj
+        if x.dim() == 2 and kernels.linear_silu_pays(x.shape[0], self.inter) and g.bias is None and \
+                kernels.plain_linear(g) and kernels.linear_silu_supported(x, g.weight):
+            return self.down_proj(kernels.linear_silu(x, g.weight))
+        return self.down_proj(kernels.silu_mul(g(x)))
 
 
 class DecoderLayer(nn.Module):

@@ -109,54 +109,35 @@ def _round_up(n: int, m: int) -> int:
     return -(-n // m) * m
 
 
-def _with_spare_rows(p: torch.Tensor, rows: int) -> torch.Tensor:
-    """p extended to `rows` rows where its storage holds that many behind it, else p."""
-    spare = p.is_contiguous() and \
-        p.untyped_storage().nbytes() // p.element_size() >= p.storage_offset() + rows * p.stride(0)
-    return p.as_strided((rows, *p.shape[1:]), p.stride()) if spare else p
-
-
 class VisionMLP(nn.Module):
-    """SwiGLU with biases (models/qwen2_5_vl.py:219-243); SiLU-and-multiply as one kernel.
+    """SwiGLU with biases (models/qwen2_5_vl.py:219-243).
 
     The published width, 3420, is no multiple of the GEMM tiles (6840 gate and up columns) nor of
-    16 bytes (3420 down-projection inputs).  gate_up_proj's parameters therefore sit at the head of
-    storage that goes on to a multiple of 256 rows, and the product runs over the spare rows too:
-    their output columns, whatever they hold, are never read (42196 rows: 596 against 658 us; 4096:
-    58.5 against 79).  A module whose parameters were replaced or copied without the spare rows runs
-    the plain product.  The down projection of PAD_ROWS rows or more runs over K padded with
-    zeros to a multiple of 128: SiLU-and-multiply writes the padded rows, the weight is copied per
-    call, so that it is the parameter's present value (42196 rows: 339 against 433 us, 4096: 38 against
-    57, 1000: 21 against 30; the copy takes about 5).
+    16 bytes (3420 down-projection inputs).  From FUSED_ROWS rows on, the gate/up projection and
+    SiLU-and-multiply run as one kernel (42196 rows: 647 us against 658 + 160, 4096: 72 against 79 + 18;
+    1000: 37 against 33), which writes its rows padded with zeros to a multiple of 128, and the down
+    projection runs over the padded K.  Its weight is copied to padded rows per call, so that it is
+    the parameter's present value (42196 rows: 339 us against 433, 4096: 38 against 57; the copy
+    takes about 5).
     """
 
-    PAD_ROWS = 1024
+    FUSED_ROWS = 1280
 
     def __init__(self, dim: int, inter: int):
         super().__init__()
         self.inter = inter
         self.gate_up_proj = nn.Linear(dim, 2 * inter, bias=True)
         self.down_proj = nn.Linear(inter, dim, bias=True)
-        rows = _round_up(2 * inter, 256)
-        self.gate_up_rows = rows if rows - 2 * inter <= 2 * inter // 32 else 2 * inter  # at most 3 % more work
-        if self.gate_up_rows != 2 * inter:
-            for name, p in list(self.gate_up_proj.named_parameters()):
-                home = p.new_empty(self.gate_up_rows, *p.shape[1:])
-                with torch.no_grad():
-                    home[:2 * inter].copy_(p)
-                setattr(self.gate_up_proj, name, nn.Parameter(home[:2 * inter]))
 
     def forward(self, x):
-        w, b = self.gate_up_proj.weight, self.gate_up_proj.bias
-        wide, wide_b = _with_spare_rows(w, self.gate_up_rows), _with_spare_rows(b, self.gate_up_rows)
-        if wide.shape[0] == wide_b.shape[0]:
-            w, b = wide, wide_b
-        gate_up = F.linear(x, w, b)[..., :2 * self.inter]
-        if self.inter % 8 == 4 and x.dim() == 2 and x.shape[0] >= self.PAD_ROWS:
-            k = _round_up(self.inter, 128)
-            return F.linear(kernels.silu_mul_padded(gate_up, k), kernels.pad_rows(self.down_proj.weight, k),
-                            self.down_proj.bias)
-        return self.down_proj(kernels.silu_mul(gate_up))
+        g, d = self.gate_up_proj, self.down_proj
+        if x.dim() == 2 and x.shape[0] >= self.FUSED_ROWS and kernels.plain_linear(g) and \
+                kernels.linear_silu_supported(x, g.weight, g.bias):
+            if self.inter % 8 == 4 and kernels.plain_linear(d):
+                k = _round_up(self.inter, 128)
+                return F.linear(kernels.linear_silu(x, g.weight, g.bias, k), kernels.pad_rows(d.weight, k), d.bias)
+            return d(kernels.linear_silu(x, g.weight, g.bias))
+        return d(kernels.silu_mul(g(x)))
 
 
 class VisionAttention(nn.Module):
