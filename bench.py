@@ -656,8 +656,6 @@ def run_vision(reps: int = 5):
     lay = run.layout
     n, h, hd = lay.num_patches, vt.cfg.num_heads, vt.head_dim
     qkv = torch.randn(n, 3 * h * hd, generator=g, device=dev, dtype=torch.bfloat16)
-    heads = kernels.vision_rope_pad(qkv, run.pos_hw, run.cos, run.sin, h, hd)
-    o = torch.empty(n, h, kernels.HEAD_DIM, dtype=torch.bfloat16, device=dev)
 
     def med_ms(fn, k=20):
         fn()
@@ -670,36 +668,34 @@ def run_vision(reps: int = 5):
         torch.cuda.synchronize()
         return sorted(a.elapsed_time(b) for a, b in e)[k // 2]
 
-    rope_ms = med_ms(lambda: kernels.vision_rope_pad(qkv, run.pos_hw, run.cos, run.sin, h, hd, out=heads))
-    rope_bytes = n * (3 * h * hd * 2 + 3 * h * kernels.HEAD_DIM * 2)
+    rope_ms = med_ms(lambda: kernels.vision_rope_(qkv, run.pos_hw, run.cos, run.sin, h, hd))
+    rope_bytes = n * 2 * (2 * h * hd * 2)  # q and k read and written in place
 
     def window():  # rotary, attention and head layout of a window block in one launch
         kernels.vision_window_attention(qkv, run.pos_hw, run.cos, run.sin, run.cu_window_host, run.cu_window, h,
                                         hd ** -0.5)
 
-    def whole():
-        kernels.varlen_attention(heads[:, 0], heads[:, 1], heads[:, 2], run.cu_full, run.cu_full, hd ** -0.5,
-                                 causal=False, plan=run.plan_full, out=o, head_dim=run.attn_head_dim)
+    def whole():  # attention over the rotated projection's rows
+        kernels.vision_attention(qkv, h, hd ** -0.5, run.plan_full)
 
     out = {"workload": "Qwen2.5-VL vision tower (public config, random init), one 4K image: grid (1, 154, 274), "
                        "42196 patches -> 10549 tokens",
            "forward_ms": round(fwd, 2), "timing": f"HIP events, median of {reps} forwards after 1 warm-up",
-           "rope_pad": {"ms": round(rope_ms, 4), "bytes": rope_bytes,
+           "rope": {"ms": round(rope_ms, 4), "bytes": rope_bytes,
                         "gbps": round(rope_bytes / (rope_ms * 1e-3) / 1e9, 1),
                         "frac_hbm_peak": round(rope_bytes / (rope_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)}}
-    # bytes each moves at least: q, k and v read, the output written (whole image: 128-element head rows)
-    for name, cu_host, fn, row in (("window_attention", lay.cu_window, window, hd),
-                                   ("whole_image_attention", lay.cu_full, whole, kernels.HEAD_DIM)):
+    for name, cu_host, fn in (("window_attention", lay.cu_window, window),
+                              ("whole_image_attention", lay.cu_full, whole)):
         ms = med_ms(fn)
         pairs = sum((b - a) ** 2 for a, b in zip(cu_host, cu_host[1:]))
         tf = 4.0 * pairs * hd * h / (ms * 1e-3) / 1e12
-        nbytes = 4 * n * h * row * 2
+        nbytes = 4 * n * h * hd * 2  # q, k and v read, the output written
         out[name] = {"ms": round(ms, 4), "sequences": len(cu_host) - 1,
                      "kernel_head_dim": run.attn_head_dim, "tflops": round(tf, 1),
                      "frac_mfma_peak": round(tf / MFMA_BF16_PEAK_TFLOPS, 4),
                      "gbps": round(nbytes / (ms * 1e-3) / 1e9, 1),
                      "frac_hbm_peak": round(nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)}
-    del vt, heads, o, qkv
+    del vt, qkv
     torch.cuda.empty_cache()
     return out
 

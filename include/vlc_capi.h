@@ -301,6 +301,28 @@ int vlc_vision_rope_pad(const void* qkv, int64_t qkv_row_stride, const int32_t* 
                         void* out, int64_t out_row_stride, void* stream);
 
 /*
+ * Vision tower: the rotation of vlc_vision_rope_pad inside the projection's rows: q and k heads are
+ * rotated in place, v stays.  Operands as there; head_dim % 16 == 0, at most 128.
+ */
+int vlc_vision_rope(void* qkv, int64_t qkv_row_stride, const int32_t* pos_hw, const void* cos_table,
+                    const void* sin_table, int64_t max_pos, int64_t num_tokens, int num_heads, int head_dim,
+                    void* stream);
+
+/*
+ * Vision tower: non-causal attention over the (rotated) QKV projection's own rows,
+ * [num_tokens, 3 * num_heads * 80] bf16 at row stride qkv_row_stride, heads 80 elements apart
+ * (flash_attn_varlen_func(..., causal=False) at models/qwen2_5_vl.py:200-210).
+ * plan_host / plan_dev: a vlc_attn_plan for num_seqs sequences, num_heads query and kv heads, head_dim
+ *   80, causal 0, the same boundaries for queries and keys, all within num_tokens.
+ * out: [num_tokens, num_heads, 80] bf16 at row stride out_row_stride; workspace as vlc_varlen_attn_fwd.
+ * head_dim: 80 (VLC_ERR_UNSUPPORTED otherwise).  qkv, out and their row strides 16-byte aligned.
+ */
+int vlc_vision_attn(const void* qkv, int64_t qkv_row_stride, int num_heads, int head_dim, int num_seqs,
+                    int64_t num_tokens, float softmax_scale, const int32_t* plan_host, const int32_t* plan_dev,
+                    int64_t plan_len, void* out, int64_t out_row_stride, void* workspace,
+                    int64_t workspace_bytes, void* stream);
+
+/*
  * Vision tower: the whole attention of a block that attends within windows, from the QKV
  * projection's rows to the output projection's input: 2-D rotary of q and k (as
  * vlc_vision_rope_pad), non-causal attention within each window, heads written unpadded.

@@ -379,3 +379,43 @@ def test_vision_mlp_fused_products(dev, rows):
         part.register_forward_hook(lambda *a: calls.append(1))
     check(mlp, "hooked")
     assert len(calls) == 2
+
+
+@pytest.mark.parametrize("grids", [[(1, 2, 2)], [(1, 4, 4), (1, 20, 34), (2, 6, 10)], [(1, 16, 16)], [(1, 60, 66)]],
+                         ids=["four", "three", "tiles", "split"])
+def test_packed_attention(dev, grids):
+    """vlc_vision_rope bit for bit against the oracle's rotation, v untouched, and vlc_vision_attn over the
+    projection's own rows against the fp32 oracle, whole images and windows: sequences of 4 to 3960 keys
+    (key counts off the 64-key tile, items that are split over the keys and merged), scores around 0 and around
+    60 (the row sum comes out of the products: rescaled with them), rows with a gap that holds NaN."""
+    say(f"vision: packed attention grids={grids}")
+    lay, qkv, cos, sin = _rope_inputs(dev, grids, seed=23)
+    n = lay.num_patches
+    ph, pw = torch.from_numpy(lay.pos_hw[:, 0]).long(), torch.from_numpy(lay.pos_hw[:, 1]).long()
+    c, s = cos.cpu(), sin.cpu()
+    c80, s80 = torch.cat((c[ph], c[pw]) * 2, -1), torch.cat((s[ph], s[pw]) * 2, -1)
+    for gain in (1.0, 8.0):
+        scaled = qkv.clone()
+        scaled[:, :1280] *= gain
+        q, k, v = scaled.reshape(n, 3, 16, 80).unbind(1)
+        q, k = ov.rope_bf16(q, c80, s80), ov.rope_bf16(k, c80, s80)
+        wide = torch.full((n, 3 * 1280 + 8), float("nan"), dtype=torch.bfloat16, device=dev)
+        wide[:, :-8] = scaled.to(dev)
+        rows = kernels.vision_rope_(wide[:, :-8], torch.from_numpy(lay.pos_hw).to(dev), cos, sin, 16, 80)
+        for part, ref in enumerate((q, k, v)):
+            got = rows.cpu().reshape(n, 3, 16, 80)[:, part]
+            assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16)), part
+        for cu in (lay.cu_full, lay.cu_window):
+            plan = kernels.plan_attention(cu, cu, 16, 16, 80, False, dev)
+            o = kernels.vision_attention(rows, 16, 80 ** -0.5, plan)
+            ref = oattn.varlen_attention(q, k, v, cu, cu, 80 ** -0.5, False)
+            assert_attn_close(o.cpu().view(n, 16, 80), ref, what=f"packed attention, {plan.num_combine} merges")
+
+
+def test_packed_attention_refuses_foreign_plans(dev):
+    """Host checks only: boundaries past the rows, another head count, another head_dim."""
+    qkv = torch.zeros(64, 3 * 1280, dtype=torch.bfloat16, device=dev)
+    for cu, heads, hd in (([0, 128], 16, 80), ([0, 64], 8, 80), ([0, 64], 16, 128)):
+        plan = kernels.plan_attention(cu, cu, heads, heads, hd, False, dev)
+        with pytest.raises((RuntimeError, ValueError)):
+            kernels.vision_attention(qkv, 16, 0.1, plan)

@@ -48,6 +48,8 @@ SIGNATURES = {
         [vp, i64, vp, vp, i64, i32, i64, vp, i64, i32, vp, i32, i32, i32, i32, f32, i32, i32, i32, vp, i64, vp],
     ),
     "vlc_vision_rope_pad": (i32, [vp, i64, vp, vp, vp, i64, i64, i32, i32, i32, vp, i64, vp]),
+    "vlc_vision_rope": (i32, [vp, i64, vp, vp, vp, i64, i64, i32, i32, vp]),
+    "vlc_vision_attn": (i32, [vp, i64, i32, i32, i32, i64, f32, vp, vp, i64, vp, i64, vp, i64, vp]),
     "vlc_vision_window_attn": (i32, [vp, i64, vp, vp, vp, i64, vp, vp, i32, i64, i32, i32, f32, vp, i64, vp]),
     "vlc_rms_norm": (i32, [vp, i64, vp, i64, vp, i64, vp, f32, i64, i64, vp, i64, vp]),
     "vlc_silu_mul": (i32, [vp, i64, i64, i64, vp, i64, vp]),

@@ -65,6 +65,7 @@ struct Params {
   int64_t out_row_stride;
   int64_t num_blocks;
   int page_size;
+  int head_stride;  // elements from one head of a row of out to the next: kHeadDim, or 80 (PACKED)
   int group;
   int causal;
   int prio_mode;  // the plan's kPPrio
@@ -124,6 +125,20 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t 
                : "s"(lds), "v"(voff), "s"(base)
                : "m0");
 }
+// The same for the lanes of `mask` only (the whole wave is active around it).
+__device__ __forceinline__ void dma16_lanes(uint64_t mask, const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
+               :
+               : "s"(lds), "v"(voff), "s"(base), "s"(mask)
+               : "m0");
+}
+// Lanes of tile-load instruction j whose chunk, (lane % 16) ^ ((lane / 16) << 2) ^ j, is below n.
+constexpr uint64_t chunk_lanes(int j, int n) {
+  uint64_t m = 0;
+  for (int i = 0; i < 64; ++i)
+    if (((i & 15) ^ ((i >> 4) << 2) ^ j) < n) m |= (uint64_t)1 << i;
+  return m;
+}
 // Per-lane 64-bit address.
 __device__ __forceinline__ void dma16_addr(const void* addr, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
@@ -169,10 +184,20 @@ __device__ __forceinline__ float half_wave_max(float x) {
 // 80..95 take v's values there).
 // AHEAD (kPagedTiles only): read the block ids of a step's tiles one step early; see
 // the launch for where it is used.
-template <int MODE, int KS = 8, int MB = 4, bool AHEAD = false>
+// PACKED (80-dim heads): the heads of q, k, v and out are 80 elements apart instead of 128, as the
+// QKV projection leaves them, and the tile loads fetch only the ten chunks a head has.  Chunk 10 of
+// every V row in LDS holds a one and zeros throughout, so dim 80 of O^T += V^T P^T is the row sum of
+// the probabilities: the 32 adds a tile that the VALU, which bounds 80-dim heads, would spend on it
+// ride on products that run over dims 64..95 anyway (fp32 sums of the bf16 P that also weigh V).  A 4K
+// image's whole-image block with it 12465 us, 13650 with the padded form, its rotary kernel (160 us a
+// block against 80) and its unpadding copy (46 us); the error against 64 bits is the same.
+template <int MODE, int KS = 8, int MB = 4, bool AHEAD = false, bool PACKED = false>
 __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const Params p) {
   constexpr bool kAheadSrc = MODE == kPagedTiles && AHEAD;
   static_assert(KS >= 1 && KS <= 8 && MB >= 1 && MB <= 4 && 2 * MB >= KS, "head_dim <= 128");
+  static_assert(!PACKED || (MODE == kContiguous && KS == 5 && MB == 3), "the packed form is the 80-dim one");
+  constexpr int kHeadStride = PACKED ? kHeadDimNarrow : kHeadDim;  // elements between the heads of a row
+  constexpr int kChunks = PACKED ? 2 * KS : 16;  // 16-byte chunks of a head row that are loaded and stored
   constexpr int NPV = 4 * MB;       // O^T += V^T P^T MFMAs per tile
   constexpr int NQK = 2 * KS;       // S^T = K Q^T MFMAs per tile
   constexpr int NU = NPV + NQK;     // units of a pipelined step
@@ -211,7 +236,7 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
   // Invalid columns load row 0 (always readable) and are zeroed.
   bf16x8 qf[KS];
   {
-    const uint16_t* qrow = p.q + (valid ? (int64_t)(q0 + qpos) * p.q_row_stride + (int64_t)head * kHeadDim : 0) +
+    const uint16_t* qrow = p.q + (valid ? (int64_t)(q0 + qpos) * p.q_row_stride + (int64_t)head * kHeadStride : 0) +
                            8 * hf;
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) {
@@ -261,13 +286,21 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
   // ---- tile loads: wave w fills rows 16w .. 16w+15, 4 rows per instruction -----
   // Lane i writes LDS slot i%16 of row 16w + 4j + i/16, so it loads that row's
   // chunk (i%16) ^ swz(row) = (i%16) ^ ((i/16) << 2) ^ j.
-  const char* kcol = reinterpret_cast<const char*>(p.k + (int64_t)g * kHeadDim);
-  const char* vcol = reinterpret_cast<const char*>(p.v + (int64_t)g * kHeadDim);
+  const char* kcol = reinterpret_cast<const char*>(p.k + (int64_t)g * kHeadStride);
+  const char* vcol = reinterpret_cast<const char*>(p.v + (int64_t)g * kHeadStride);
   const int64_t kst = p.k_row_stride * 2, vst = p.v_row_stride * 2;  // bytes
   const uint32_t lrow0 = 16 * wave + (lane >> 4);
   const uint32_t lchunk0 = (uint32_t)((lane & 15) ^ ((lane >> 4) << 2));
   const char* zero = reinterpret_cast<const char*>(kZeroRow);
 
+  uint64_t lanes[4];  // PACKED: the lanes of each tile-load instruction whose chunk a head has
+  if constexpr (PACKED) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lanes[j] = chunk_lanes(j, kChunks);
+      asm volatile("" : "+s"(lanes[j]));  // kept in scalar registers
+    }
+  }
   // ---- state ---------------------------------------------------------------------
   f32x16 o[4];
 #pragma unroll
@@ -478,8 +511,10 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
       float pe = fast_exp2(__builtin_fmaf(get(n), p.scale_log2, -m_base));
       pin(pe);
       set(n, pe);
-      if (n > 0) rs += pend;
-      pend = pe;
+      if constexpr (!PACKED) {
+        if (n > 0) rs += pend;
+        pend = pe;
+      }
     };
 
     // exp2 slices: units 4 .. 4 + kTwo - 1 take two elements each, the rest one, so the
@@ -493,7 +528,16 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
       if (i + kAhead < NU) read_op(i + kAhead);
       mfma_op(i);
       // row (< 64) x row stride (< 2^24 bytes, checked on the host): a 24-bit multiply-add
-      if (i < 4) {
+      if constexpr (PACKED) {
+        if (i < 4) {
+          dma16_lanes(lanes[i], dk.base, __umul24(min(lr + 4 * i, dk.last), (uint32_t)kst) + ((lcn ^ (uint32_t)i) << 4),
+                      lds_u32(k_ld + (16 * wave + 4 * i) * 256));
+        } else if (i < 8) {
+          const int r = i - 4;
+          dma16_lanes(lanes[r], dv.base, __umul24(min(lr + 4 * r, dv.last), (uint32_t)vst) + ((lcn ^ (uint32_t)r) << 4),
+                      lds_u32(v_ld + (16 * wave + 4 * r) * 256));
+        }
+      } else if (i < 4) {
         dma16(dk.base, __umul24(min(lr + 4 * i, dk.last), (uint32_t)kst) + ((lcn ^ (uint32_t)i) << 4),
               lds_u32(k_ld + (16 * wave + 4 * i) * 256));
       } else if (i < 8) {
@@ -573,7 +617,16 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
   if (n_tiles > 0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      *reinterpret_cast<u32x4v*>(v_buf1 + (i * kThreads + tid) * 16) = u32x4v{0u, 0u, 0u, 0u};
+    {
+      const int slot16 = i * kThreads + tid;
+      u32x4v w = {0u, 0u, 0u, 0u};
+      if constexpr (PACKED) {  // chunk 10 is a one and zeros, in both V buffers; the tile loads leave it alone
+        const int row = slot16 >> 4;
+        if (((slot16 & 15) ^ swz(row)) == kChunks) w[0] = 0x3f80u;
+        *reinterpret_cast<u32x4v*>(v_buf0 + slot16 * 16) = w;
+      }
+      *reinterpret_cast<u32x4v*>(v_buf1 + slot16 * 16) = w;
+    }
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -583,8 +636,15 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t off = ((lchunk0 ^ (uint32_t)j) << 4);
-        dma16(d0.base, min(lrow0 + 4 * j, d0.last) * (uint32_t)kst + off, lds_u32(k_buf0 + (16 * wave + 4 * j) * 256));
-        dma16(d1.base, min(lrow0 + 4 * j, d1.last) * (uint32_t)kst + off, lds_u32(k_buf1 + (16 * wave + 4 * j) * 256));
+        const uint32_t o0 = min(lrow0 + 4 * j, d0.last) * (uint32_t)kst + off, o1 = min(lrow0 + 4 * j, d1.last) * (uint32_t)kst + off;
+        const uint32_t l0 = lds_u32(k_buf0 + (16 * wave + 4 * j) * 256), l1 = lds_u32(k_buf1 + (16 * wave + 4 * j) * 256);
+        if constexpr (PACKED) {
+          dma16_lanes(lanes[j], d0.base, o0, l0);
+          dma16_lanes(lanes[j], d1.base, o1, l1);
+        } else {
+          dma16(d0.base, o0, l0);
+          dma16(d1.base, o1, l1);
+        }
       }
     }
     // Paged: block ids of the item's tiles, read once into LDS (the steps take them
@@ -652,7 +712,12 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
   // writes 1 KB of contiguous memory.  The stores write through L2 (st16_wt): the
   // next kernel reads them, and dirty L2 lines would be written back between the two
   // kernels.  The K buffers are free here.
-  const float l_tot = l_run + __shfl_xor(l_run, 32);
+  // PACKED: the row sum is dim 80, row 16 of block 2, held by the lower half-wave
+  float l_tot;
+  if constexpr (PACKED)
+    l_tot = __shfl(o[2][8], lc);
+  else
+    l_tot = l_run + __shfl_xor(l_run, 32);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   uint8_t* stage = (wave < 2 ? k_buf0 : k_buf1) + (wave & 1) * (kTileK * 256 / 2);
 #pragma unroll
@@ -676,9 +741,9 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
       // A split of a longer key range writes its normalised partial in bf16 plus
       // (m, l) in fp32 to its workspace slot.
       uint16_t* dst = slot < 0 ? p.out + (int64_t)(q0 + q_start + posx) * p.out_row_stride +
-                                     (int64_t)(g * p.group + colx - posx * p.group) * kHeadDim
+                                     (int64_t)(g * p.group + colx - posx * p.group) * kHeadStride
                                : p.part_o + ((int64_t)slot * kCols + colx) * kHeadDim;
-      st16_wt(dst + 8 * ch, v);
+      if (!PACKED || ch < kChunks) st16_wt(dst + 8 * ch, v);
     }
   }
   if (slot >= 0 && valid && hf == 0)
@@ -830,7 +895,8 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(const Params p) 
   const int hh = col - pos * p.group;
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   uint16_t* orow = p.out + (int64_t)(q0 + q_start + pos) * p.out_row_stride +
-                   (int64_t)(g * p.group + hh) * kHeadDim + d;
+                   (int64_t)(g * p.group + hh) * p.head_stride + d;
+  if (d >= p.head_stride) return;  // packed heads end here
   u32x4v w;
 #pragma unroll
   for (int t = 0; t < 4; ++t) w[t] = pack_bf16x2(acc[2 * t] * inv, acc[2 * t + 1] * inv);
@@ -841,7 +907,7 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(const Params p) 
 }  // namespace attn
 }  // namespace vlc
 
-VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void* k,
+static int attn_fwd(const void* q, int64_t q_row_stride, const void* k,
                                 int64_t k_row_stride, const void* v, int64_t v_row_stride,
                                 const int32_t* block_table, int64_t bt_row_stride, int page_size,
                                 int64_t num_blocks, const int32_t* cu_seqlens_q,
@@ -849,7 +915,7 @@ VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void*
                                 int num_heads_kv, int head_dim, float softmax_scale, int causal,
                                 const int32_t* plan_host, const int32_t* plan_dev, int64_t plan_len,
                                 void* out, int64_t out_row_stride, void* workspace,
-                                int64_t workspace_bytes, void* stream) {
+                                int64_t workspace_bytes, int head_stride, void* stream) {
   using namespace vlc;
   using namespace vlc::attn;
   if (head_dim != kHeadDim && head_dim != kHeadDimNarrow) return VLC_ERR_UNSUPPORTED;
@@ -885,8 +951,8 @@ VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void*
     return VLC_ERR_INVALID;
   // tile-load offsets are 24-bit products: row (< 64) x row stride in bytes
   if (k_row_stride * 2 >= (int64_t(1) << 24) || v_row_stride * 2 >= (int64_t(1) << 24)) return VLC_ERR_UNSUPPORTED;
-  if (q_row_stride < (int64_t)num_heads_q * kHeadDim || out_row_stride < (int64_t)num_heads_q * kHeadDim ||
-      k_row_stride < (int64_t)num_heads_kv * kHeadDim || v_row_stride < (int64_t)num_heads_kv * kHeadDim)
+  if (q_row_stride < (int64_t)num_heads_q * head_stride || out_row_stride < (int64_t)num_heads_q * head_stride ||
+      k_row_stride < (int64_t)num_heads_kv * head_stride || v_row_stride < (int64_t)num_heads_kv * head_stride)
     return VLC_ERR_INVALID;
   if (block_table && (page_size <= 0 || bt_row_stride <= 0 || num_blocks <= 0)) return VLC_ERR_INVALID;
   // Paged K/V: a wave loads 16 consecutive keys of a tile, which must share a page.
@@ -915,6 +981,7 @@ VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void*
   prm.out_row_stride = out_row_stride;
   prm.num_blocks = num_blocks;
   prm.page_size = block_table ? page_size : 1;
+  prm.head_stride = head_stride;
   prm.group = group;
   prm.causal = causal ? 1 : 0;
   prm.prio_mode = h[kPPrio];
@@ -922,7 +989,10 @@ VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void*
 
   hipStream_t s = as_stream(stream);
   const int mode = !block_table ? kContiguous : (page_size % kTileK == 0 ? kPagedTiles : kPagedRows);
-  if (head_dim == kHeadDimNarrow)
+  if (head_stride == kHeadDimNarrow)
+    hipLaunchKernelGGL((attn_fwd_kernel<kContiguous, kHeadDimNarrow / 16, (kHeadDimNarrow + 31) / 32, false, true>),
+                       dim3((unsigned)n_items), dim3(kThreads), 0, s, prm);
+  else if (head_dim == kHeadDimNarrow)
     hipLaunchKernelGGL((attn_fwd_kernel<kContiguous, kHeadDimNarrow / 16, (kHeadDimNarrow + 31) / 32>),
                        dim3((unsigned)n_items), dim3(kThreads), 0, s, prm);
   else if (mode == kContiguous)
@@ -948,4 +1018,41 @@ VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void*
     st = launch_status();
   }
   return st;
+}
+
+VLC_API int vlc_varlen_attn_fwd(const void* q, int64_t q_row_stride, const void* k,
+                                int64_t k_row_stride, const void* v, int64_t v_row_stride,
+                                const int32_t* block_table, int64_t bt_row_stride, int page_size,
+                                int64_t num_blocks, const int32_t* cu_seqlens_q,
+                                const int32_t* cu_seqlens_k, int num_seqs, int num_heads_q,
+                                int num_heads_kv, int head_dim, float softmax_scale, int causal,
+                                const int32_t* plan_host, const int32_t* plan_dev, int64_t plan_len,
+                                void* out, int64_t out_row_stride, void* workspace,
+                                int64_t workspace_bytes, void* stream) {
+  return attn_fwd(q, q_row_stride, k, k_row_stride, v, v_row_stride, block_table, bt_row_stride, page_size, num_blocks, cu_seqlens_q,
+                  cu_seqlens_k, num_seqs, num_heads_q, num_heads_kv, head_dim, softmax_scale, causal, plan_host, plan_dev,
+                  plan_len, out, out_row_stride, workspace, workspace_bytes, vlc::attn::kHeadDim,
+                  stream);
+}
+
+VLC_API int vlc_vision_attn(const void* qkv, int64_t qkv_row_stride, int num_heads, int head_dim, int num_seqs,
+                            int64_t num_tokens, float softmax_scale, const int32_t* plan_host, const int32_t* plan_dev,
+                            int64_t plan_len, void* out, int64_t out_row_stride, void* workspace,
+                            int64_t workspace_bytes, void* stream) {
+  using namespace vlc::attn;
+  if (head_dim != kHeadDimNarrow) return VLC_ERR_UNSUPPORTED;
+  const int64_t width = (int64_t)num_heads * kHeadDimNarrow;
+  if (num_heads <= 0 || qkv_row_stride < 3 * width || num_tokens < 0) return VLC_ERR_INVALID;
+  if (!qkv || !plan_host || !plan_dev || plan_len < kHeaderInts) return VLC_ERR_PLAN;
+  if (plan_len < kHeaderInts + ((int64_t)plan_host[kPNumItems] + plan_host[kPNumCombine]) * kItemInts) return VLC_ERR_PLAN;
+  for (int64_t i = 0; i < plan_host[kPNumItems]; ++i) {  // the boundaries the kernel reads and writes by
+    const int32_t* v = plan_host + kHeaderInts + i * kItemInts;
+    if (v[7] < 0 || v[8] < 0 || (int64_t)v[7] + v[8] > num_tokens || v[9] < 0 || v[10] < 0 ||
+        (int64_t)v[9] + v[10] > num_tokens || (int64_t)v[2] + v[3] > v[8])
+      return VLC_ERR_PLAN;
+  }
+  const char* rows = static_cast<const char*>(qkv);
+  return attn_fwd(rows, qkv_row_stride, rows + width * 2, qkv_row_stride, rows + width * 4, qkv_row_stride, nullptr, 0, 0,
+                  0, nullptr, nullptr, num_seqs, num_heads, num_heads, head_dim, softmax_scale, 0, plan_host, plan_dev,
+                  plan_len, out, out_row_stride, workspace, workspace_bytes, kHeadDimNarrow, stream);
 }

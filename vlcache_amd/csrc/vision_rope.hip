@@ -96,8 +96,73 @@ __global__ __launch_bounds__(kThreads) void vision_rope_pad_kernel(
   *dst = u32x4{ys[0], ys[1], ys[2], ys[3]};
 }
 
+// The same rotation of q and k inside the projection's rows (v stays): a lane owns a pair of
+// chunks, dims [8c, 8c + 8) and [half + 8c, ...), of one head, so it reads nothing that another lane
+// writes.  Bound by memory: q and k read and written once, 432 MB for a 4K image, where the padded
+// split reads q, k, v and writes 1.6 times as much (843 MB, 160 us).
+__global__ __launch_bounds__(kThreads) void vision_rope_kernel(
+    char* __restrict__ qkv, int64_t qkv_stride_b, const int32_t* __restrict__ pos_hw,
+    const uint16_t* __restrict__ cos_tab, const uint16_t* __restrict__ sin_tab, int max_pos, int num_heads,
+    int head_dim, uint32_t units, uint32_t per_token) {
+  const uint32_t u = blockIdx.x * kThreads + threadIdx.x;
+  if (u >= units) return;
+  const int half = head_dim >> 1, quarter = head_dim >> 2, chunks = half >> 3;
+  const uint32_t n = u / per_token, x = u - n * per_token;
+  const int hp = x / chunks, a0 = (x - hp * chunks) * 8;  // head of q, then of k; first rotation pair
+  char* row = qkv + n * qkv_stride_b + ((int64_t)hp * head_dim + a0) * 2;
+  const u32x4 lo = *reinterpret_cast<const u32x4*>(row), hi = *reinterpret_cast<const u32x4*>(row + half * 2);
+  int ph = pos_hw[2 * (int64_t)n], pw = pos_hw[2 * (int64_t)n + 1];
+  ph = ph < 0 ? 0 : (ph >= max_pos ? max_pos - 1 : ph);
+  pw = pw < 0 ? 0 : (pw >= max_pos ? max_pos - 1 : pw);
+  uint32_t cw[4], sw[4];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int a = a0 + 4 * r;
+    const int t = a < quarter ? ph * quarter + a : pw * quarter + (a - quarter);
+    const uint2 cv = ld4(cos_tab + t), sv = ld4(sin_tab + t);
+    cw[2 * r] = cv.x, cw[2 * r + 1] = cv.y;
+    sw[2 * r] = sv.x, sw[2 * r + 1] = sv.y;
+  }
+  const uint32_t ls[4] = {lo.x, lo.y, lo.z, lo.w}, hs[4] = {hi.x, hi.y, hi.z, hi.w};
+  uint32_t yl[4], yh[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    yl[w] = yh[w] = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float cs = bf16_bits_to_f32((cw[w] >> (16 * h)) & 0xffffu), sn = bf16_bits_to_f32((sw[w] >> (16 * h)) & 0xffffu);
+      const float a = bf16_bits_to_f32((ls[w] >> (16 * h)) & 0xffffu), b = bf16_bits_to_f32((hs[w] >> (16 * h)) & 0xffffu);
+      yl[w] |= f32_to_bf16_bits(rbf(a * cs) + rbf(-b * sn)) << (16 * h);
+      yh[w] |= f32_to_bf16_bits(rbf(b * cs) + rbf(a * sn)) << (16 * h);
+    }
+  }
+  *reinterpret_cast<u32x4*>(row) = u32x4{yl[0], yl[1], yl[2], yl[3]};
+  *reinterpret_cast<u32x4*>(row + half * 2) = u32x4{yh[0], yh[1], yh[2], yh[3]};
+}
+
 }  // namespace
 }  // namespace vlc
+
+VLC_API int vlc_vision_rope(void* qkv, int64_t qkv_row_stride, const int32_t* pos_hw, const void* cos_table,
+                            const void* sin_table, int64_t max_pos, int64_t num_tokens, int num_heads, int head_dim,
+                            void* stream) {
+  using namespace vlc;
+  if (num_tokens < 0 || num_heads <= 0 || head_dim <= 0 || head_dim % 16 != 0 || head_dim > 128 || max_pos <= 0 ||
+      max_pos >= (1 << 24) || qkv_row_stride < 3 * (int64_t)num_heads * head_dim)
+    return VLC_ERR_INVALID;
+  if (num_tokens == 0) return VLC_OK;
+  if (!qkv || !pos_hw || !cos_table || !sin_table) return VLC_ERR_INVALID;
+  const int64_t per_token = 2 * (int64_t)num_heads * (head_dim / 16), units = num_tokens * per_token;
+  if (!aligned16(qkv) || qkv_row_stride % 8 || (reinterpret_cast<uintptr_t>(cos_table) & 7) ||
+      (reinterpret_cast<uintptr_t>(sin_table) & 7) || units >= ((int64_t)1 << 31) ||
+      (int64_t)(head_dim / 4) * max_pos >= ((int64_t)1 << 31))
+    return VLC_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(vision_rope_kernel, dim3((unsigned)((units + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                     as_stream(stream), static_cast<char*>(qkv), qkv_row_stride * 2, pos_hw,
+                     static_cast<const uint16_t*>(cos_table), static_cast<const uint16_t*>(sin_table), (int)max_pos,
+                     num_heads, head_dim, (uint32_t)units, (uint32_t)per_token);
+  return launch_status();
+}
 
 VLC_API int vlc_vision_rope_pad(const void* qkv, int64_t qkv_row_stride, const int32_t* pos_hw,
                                 const void* cos_table, const void* sin_table, int64_t max_pos,

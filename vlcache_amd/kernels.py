@@ -608,6 +608,38 @@ def vision_rope_pad(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Te
     return out
 
 
+def vision_rope_(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.Tensor,
+                 num_heads: int, head_dim: int) -> torch.Tensor:
+    """vision_rope_pad's rotation of q and k inside qkv's rows (vlc_vision_rope); returns qkv."""
+    _require_device("vision_rope_", qkv, pos_hw, cos_table, sin_table)
+    _check_vision_rows(qkv, pos_hw, cos_table, sin_table, num_heads, head_dim)
+    st = _lib.load().vlc_vision_rope(qkv.data_ptr(), qkv.stride(0), pos_hw.data_ptr(), cos_table.data_ptr(),
+                                     sin_table.data_ptr(), cos_table.shape[0], qkv.shape[0], num_heads, head_dim,
+                                     _stream(qkv))
+    _lib.check("vlc_vision_rope", st)
+    return qkv
+
+
+def vision_attention(qkv: torch.Tensor, num_heads: int, softmax_scale: float, plan: AttnPlan) -> torch.Tensor:
+    """Non-causal attention over rotated QKV rows [N, 3 * num_heads * 80] with plan's boundaries
+    (vlc_vision_attn) -> [N, num_heads * 80]."""
+    _require_device("vision_attention", qkv)
+    n, width = qkv.shape[0], num_heads * VISION_HEAD_DIM
+    if qkv.dtype != torch.bfloat16 or qkv.dim() != 2 or qkv.shape[1] != 3 * width or qkv.stride(1) != 1:
+        raise ValueError(f"qkv must be bf16 [N, {3 * width}] with contiguous rows")
+    if plan.num_heads_q != num_heads or plan.num_heads_kv != num_heads or plan.causal or \
+            plan.host[_PLAN_HEAD_DIM] != VISION_HEAD_DIM:
+        raise ValueError("attention plan does not match the call")
+    out = torch.empty(n, width, dtype=torch.bfloat16, device=qkv.device)
+    ws = plan.workspace
+    st = _lib.load().vlc_vision_attn(
+        qkv.data_ptr(), qkv.stride(0), num_heads, VISION_HEAD_DIM, plan.num_seqs, n, float(softmax_scale),
+        plan.host.__array_interface__["data"][0], plan.dev.data_ptr(), plan.host.size, out.data_ptr(), width,
+        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream(qkv))
+    _lib.check("vlc_vision_attn", st)
+    return out
+
+
 def vision_window_attention(qkv: torch.Tensor, pos_hw: torch.Tensor, cos_table: torch.Tensor,
                             sin_table: torch.Tensor, cu_host: np.ndarray, cu_dev: torch.Tensor, num_heads: int,
                             softmax_scale: float) -> torch.Tensor:

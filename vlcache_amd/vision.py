@@ -10,15 +10,17 @@ On gfx950:
   * the window layout (window order, window and image boundaries, patch
     positions) is integer host work, vectorised with numpy, computed once per
     batch of images;
-  * each block's q/k rotation and the split of the QKV projection into
-    128-dim head rows run as one kernel (vlc_vision_rope_pad);
-  * attention runs on the varlen attention kernel in its contiguous,
-    non-causal mode (the reference calls flash_attn_varlen_func with
-    causal=False and cu_seqlens_q == cu_seqlens_k, :200-210), in its 80-dim
-    variant: heads stay zero-padded 128-element rows, the products skip the
-    padding; one work plan per boundary list serves every block;
-  * each RMSNorm (with its residual add) and the MLP's SiLU-and-multiply run
-    as one kernel each; GEMMs and the merger's GELU run on torch (hipBLASLt).
+  * a block that attends within windows of at most 64 patches with 80-dim heads runs its
+    rotation, attention and head layout as one kernel (vlc_vision_window_attn);
+  * other blocks with 80-dim heads rotate q and k inside the projection's rows
+    (vlc_vision_rope) and attend over those rows (vlc_vision_attn; the reference calls
+    flash_attn_varlen_func with causal=False and cu_seqlens_q == cu_seqlens_k, :200-210);
+    one work plan per boundary list serves every block;
+  * other head widths split the projection into zero-padded 128-dim head rows
+    (vlc_vision_rope_pad) for the general attention kernel;
+  * each RMSNorm (with its residual add) runs as one kernel, the MLP's gate/up projection
+    with SiLU-and-multiply as one for many rows (vlc_linear_silu); the other GEMMs and the
+    merger's GELU run on torch (hipBLASLt).
 
 As in the reference, the rotary angles are rounded to bf16 before cos/sin
 (:486-487) and the rotation itself is bf16 arithmetic.  The Conv3d patch
@@ -158,8 +160,11 @@ class VisionAttention(nn.Module):
         if not full and run.fused_windows:
             return self.proj(kernels.vision_window_attention(qkv, run.pos_hw, run.cos, run.sin, run.cu_window_host,
                                                              run.cu_window, self.num_heads, self.head_dim ** -0.5))
-        heads = kernels.vision_rope_pad(qkv, run.pos_hw, run.cos, run.sin, self.num_heads, self.head_dim)
         cu, plan = (run.cu_full, run.plan_full) if full else (run.cu_window, run.plan_window)
+        if self.head_dim == kernels.VISION_HEAD_DIM:
+            kernels.vision_rope_(qkv, run.pos_hw, run.cos, run.sin, self.num_heads, self.head_dim)
+            return self.proj(kernels.vision_attention(qkv, self.num_heads, self.head_dim ** -0.5, plan))
+        heads = kernels.vision_rope_pad(qkv, run.pos_hw, run.cos, run.sin, self.num_heads, self.head_dim)
         o = kernels.varlen_attention(heads[:, 0], heads[:, 1], heads[:, 2], cu, cu, self.head_dim ** -0.5,
                                      causal=False, plan=plan, head_dim=run.attn_head_dim)
         return self.proj(o[..., :self.head_dim].reshape(n, self.num_heads * self.head_dim))
