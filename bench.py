@@ -618,11 +618,10 @@ def run_vision(reps: int = 5):
     whole-image attention at blocks 7/15/23/31, window 112 px).  Whole forward:
     HIP events around each of `reps` calls after one warm-up, median.  The three
     kernels of a block's attention on the same layout, each the median of 20
-    event-timed calls: the fused rotary + head padding (HBM: bytes read + written),
-    the window attention and the whole-image attention (MFMA: 4 * pairs * 80 dims
-    * 16 heads; the kernel's 80-dim variant skips the heads' zero padding; HBM: the q, k, v
-    head rows read once and the output written once, which bounds the window attention's
-    64-token windows).
+    event-timed calls: the rotary of q and k in place (HBM: bytes read + written),
+    the window blocks' rotary + attention, and the whole-image attention (MFMA: 4 * pairs
+    * 80 dims * 16 heads; HBM: the q, k, v head rows read once and the output written once,
+    which bounds the window attention's 64-token windows).
     """
     from vlcache_amd import kernels
     from vlcache_amd.config import QWEN25_VL_VISION

@@ -407,13 +407,22 @@ int vlc_linear_skinny(const void* x, int64_t x_row_stride, int64_t rows, int64_t
                       void* out, int64_t out_row_stride, void* stream);
 
 /*
+ * The gate/up projection of at most 16 rows with SiLU-and-multiply: weight holds inter gate rows, then
+ * inter up rows (no bias); out[m][i] = bf16(silu(bf16(gate)) * bf16(up)), the bits that vlc_silu_mul
+ * gives for such a gate and up.  Otherwise as vlc_linear_skinny with out_features = inter.
+ */
+int vlc_linear_skinny_silu(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
+                           const void* weight, int64_t w_row_stride, int64_t inter, void* out,
+                           int64_t out_row_stride, void* stream);
+
+/*
  * The same for at most 64 rows, K split across workgroups (long K, few features: the down
  * projection of a decode step with many sequences).  Operands as vlc_linear_skinny, with
  * out_features a multiple of 32.  workspace: device scratch of at least
- * vlc_linear_split_workspace(rows, out_features) bytes, 16-byte aligned, used by this call
+ * vlc_linear_split_workspace(rows, in_features, out_features) bytes, 16-byte aligned, used by this call
  * only; its contents before and after do not matter.
  */
-int64_t vlc_linear_split_workspace(int64_t rows, int64_t out_features);
+int64_t vlc_linear_split_workspace(int64_t rows, int64_t in_features, int64_t out_features);
 int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
                      const void* weight, int64_t w_row_stride, int64_t out_features, const void* bias,
                      void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes,

@@ -197,7 +197,8 @@ def test_linear_skinny_kernel_choice(dev, m, k, n):
 
 
 @pytest.mark.parametrize("m", [1, 17, 32, 33, 48, 49, 64])
-@pytest.mark.parametrize("k,n,bias", [(32, 32, True), (2048, 512, True), (11008, 2048, False), (4128, 8224, False)])
+@pytest.mark.parametrize("k,n,bias", [(32, 32, True), (2048, 512, True), (11008, 2048, False), (4128, 8224, False),
+                                      (4128, 3072, True), (4096, 3072, False), (4096, 3104, False)])
 def test_linear_split(dev, m, k, n, bias):
     """vlc_linear_split: row blocks' edges, fewer k steps than splits, one split only (N 8224), through
     the layer too; the bar of test_linear_skinny."""
@@ -318,3 +319,20 @@ def test_decoder_mlp_route(dev, rows, inter, pays):
         got = mlp(x).float()
         ref = mlp.down_proj(kernels.silu_mul(mlp.gate_up_proj(x))).float()
     assert (got - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("k,inter", [(32, 16), (64, 48), (128, 112), (256, 2064), (2048, 11008)])
+def test_linear_skinny_silu(dev, m, k, inter):
+    """The bits of vlc_silu_mul on vlc_linear_skinny's output, up to a gate or up whose fp32 sum (in another
+    order) rounds the other way: 2^-6 of (1 + |gate|) (1 + |up|) as in test_linear_silu, 98 % equal."""
+    from vlcache_amd import kernels
+
+    say(f"linear_skinny_silu m={m} k={k} inter={inter}")
+    x, w = randn_bf16((m, k + 8), m + k).to(dev)[:, :k], randn_bf16((2 * inter, k), inter + k, 0.05).to(dev)
+    out = kernels.linear_skinny_silu(x, w).float()
+    gu = (x.double() @ w.double().t()).float().to(torch.bfloat16)
+    ref = kernels.silu_mul(gu).float()
+    scale = (1 + gu[:, :inter].float().abs()) * (1 + gu[:, inter:].float().abs())
+    assert ((out - ref).abs() <= 2.0 ** -6 * scale).all()
+    assert float((out == ref).float().mean()) >= 0.98 or out.numel() < 200

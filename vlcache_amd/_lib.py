@@ -56,7 +56,8 @@ SIGNATURES = {
     "vlc_silu_mul_padded": (i32, [vp, i64, i64, i64, vp, i64, i64, vp]),
     "vlc_pad_rows": (i32, [vp, i64, i64, i64, vp, i64, i64, vp]),
     "vlc_linear_skinny": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, vp]),
-    "vlc_linear_split_workspace": (i64, [i64, i64]),
+    "vlc_linear_skinny_silu": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, i64, vp]),
+    "vlc_linear_split_workspace": (i64, [i64, i64, i64]),
     "vlc_linear_split": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, vp, i64, vp]),
     "vlc_linear_silu": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, i64, vp]),
     "vlc_attn_plan": (

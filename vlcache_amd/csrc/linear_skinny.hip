@@ -56,19 +56,30 @@ struct Args {
   int out_features;
 };
 
+// SiLU-and-multiply as vlc_silu_mul computes it, of a gate and an up value rounded to bf16.
+__device__ __forceinline__ float silu_mul(float gate, float up) {
+  const float g = static_cast<float>(static_cast<__bf16>(gate)), u = static_cast<float>(static_cast<__bf16>(up));
+  return g / (1.0f + expf(-g)) * u;
+}
+
 // U: k steps in flight; KS waves of the workgroup's W split K; gridDim.y splits it further.
-template <int U, int KS, int Z, int TF, int RB, int W>
+// kSilu: the second half of a tile's TF feature groups are the up rows (out_features further) of the
+// gate rows in the first half, and the output is silu(gate) * up: a decode step then has one launch
+// less per layer (four layers of the 3B model, one row: 333.6 -> 326.5 us with the logits).
+template <int U, int KS, int Z, int TF, int RB, int W, bool kSilu = false>
 __global__ __launch_bounds__(64 * W) void linear_skinny_kernel(const Args p) {
   constexpr int kTiles = W / KS;  // tiles of a workgroup
   constexpr int F = 16 / Z;       // features, and rows, of a diagonal block
   constexpr int kStepB = 64 * Z;  // bytes of a row per k step
+  constexpr int TO = kSilu ? TF / 2 : TF;  // feature groups of the output
+  static_assert(!kSilu || TF % 2 == 0, "gate and up halves");
   __shared__ float part[W][TF][RB][16 * kPad];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
   const int z = r / F, f = r % F;  // diagonal block; feature (A) or row of x (B) within it
   const int t = blockIdx.x * kTiles + wave / KS;
   const bool live = t < p.tiles;   // the last workgroup's tiles past N do no work
-  const char* wp = p.w + (int64_t)((live ? t : 0) * (F * TF) + f) * p.w_stride_b + z * 64 + g * 16;
+  const char* wp = p.w + (int64_t)((live ? t : 0) * (F * TO) + f) * p.w_stride_b + z * 64 + g * 16;
   const char* xp[RB];
   bool xr[RB];
 #pragma unroll
@@ -88,7 +99,9 @@ __global__ __launch_bounds__(64 * W) void linear_skinny_kernel(const Args p) {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
 #pragma unroll
-      for (int j = 0; j < TF; ++j) a[u][j] = ld16(wp + (int64_t)(j * F) * p.w_stride_b + (int64_t)(s0 + u) * kStepB);
+      for (int j = 0; j < TF; ++j)
+        a[u][j] = ld16(wp + (int64_t)(j % TO * F + (j >= TO ? p.out_features : 0)) * p.w_stride_b +
+                       (int64_t)(s0 + u) * kStepB);
 #pragma unroll
       for (int q = 0; q < RB; ++q) b[u][q] = xr[q] ? ld16(xp[q] + (int64_t)(s0 + u) * kStepB) : zero;
     }
@@ -112,18 +125,24 @@ __global__ __launch_bounds__(64 * W) void linear_skinny_kernel(const Args p) {
       for (int e = 0; e < 4; ++e) part[wave][j][q][(4 * g + e) * kPad + r] = acc[j][q][e];
   __syncthreads();
   // output (tile, row block, row, feature) = sum over the waves of the tile and the diagonal blocks
-  constexpr int kOut = kTiles * RB * F * TF * F;
+  constexpr int kOut = kTiles * RB * F * TO * F;
   for (int i = threadIdx.x; i < kOut; i += 64 * W) {
-    const int ff = i % F, j = i / F % TF, m = i / (F * TF) % F, q = i / (F * TF * F) % RB, tt = i / (F * TF * F * RB);
+    const int ff = i % F, j = i / F % TO, m = i / (F * TO) % F, q = i / (F * TO * F) % RB, tt = i / (F * TO * F * RB);
     const int row = m + F * q, tile = blockIdx.x * kTiles + tt;
     if (row >= p.rows || tile >= p.tiles) continue;
-    float y = 0.f;
+    auto sum = [&](int jj) __attribute__((always_inline)) {
+      float y = 0.f;
 #pragma unroll
-    for (int v = 0; v < KS; ++v)
+      for (int v = 0; v < KS; ++v)
 #pragma unroll
-      for (int zz = 0; zz < Z; ++zz) y += part[tt * KS + v][j][q][(zz * F + ff) * kPad + zz * F + m];
-    const int n = (tile * TF + j) * F + ff;
-    if (gridDim.y == 1)
+        for (int zz = 0; zz < Z; ++zz) y += part[tt * KS + v][jj][q][(zz * F + ff) * kPad + zz * F + m];
+      return y;
+    };
+    const float y = sum(j);
+    const int n = (tile * TO + j) * F + ff;
+    if constexpr (kSilu)
+      p.out[row * p.out_stride + n] = (uint16_t)f32_to_bf16_bits(silu_mul(y, sum(j + TO)));
+    else if (gridDim.y == 1)
       p.out[row * p.out_stride + n] =
           (uint16_t)f32_to_bf16_bits(p.bias ? y + bf16_bits_to_f32(p.bias[n]) : y);
     else
@@ -147,20 +166,25 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const float* __restr
   }
 }
 
-template <int U, int KS, int Z, int TF, int RB, int W>
+template <int U, int KS, int Z, int TF, int RB, int W, bool kSilu = false>
 void launch(Args a, int64_t in_features, int splits, hipStream_t st) {
   constexpr int kTiles = W / KS;
-  a.tiles = a.out_features / (16 / Z * TF);
+  a.tiles = a.out_features / (16 / Z * (kSilu ? TF / 2 : TF));
   a.k_steps = (int)(in_features / (32 * Z));
-  hipLaunchKernelGGL((linear_skinny_kernel<U, KS, Z, TF, RB, W>),
+  hipLaunchKernelGGL((linear_skinny_kernel<U, KS, Z, TF, RB, W, kSilu>),
                      dim3((unsigned)((a.tiles + kTiles - 1) / kTiles), (unsigned)splits), dim3(64 * W), 0, st, a);
 }
 
-// K splits across workgroups: one workgroup a CU (18944 x 3584, 32 rows: 43.0 us with 2 splits,
-// 46.9 with 1 or 4; 11008 x 2048: 20.1 with 4, 26 with 1).
-int num_splits(int64_t out_features) {
-  const int64_t tiles = out_features / 32;
-  const int64_t s = (256 + tiles / 2) / tiles;
+// vlc_linear_split's tile and K splits across workgroups: about one workgroup a CU.  Two or four feature
+// groups a wave re-read x less, two diagonal blocks read 128 contiguous bytes of a weight row.  us, 18944 x 3584
+// and 11008 x 2048, in brackets the library: 32 rows 38.2 (110), 18.2 (27), with tiles of 32 features and
+// one diagonal block 43.0 and 20.1; 64 rows 54.8 (91), 25.2 (31), with tiles of 32 features 63.0 and 26.9.
+int split_tile(int64_t rows, int64_t k, int64_t n) {
+  if (rows > 16 && rows <= 32 && k % 64 == 0) return n % 64 == 0 && n >= 64 * 48 ? 64 : 32;
+  return rows > 32 && n % 64 == 0 ? 64 : 32;
+}
+int num_splits(int64_t tiles) {
+  const int64_t s = 256 / tiles;
   return (int)(s < 1 ? 1 : s > 8 ? 8 : s);
 }
 
@@ -217,10 +241,35 @@ VLC_API int vlc_linear_skinny(const void* x, int64_t x_row_stride, int64_t rows,
   return launch_status();
 }
 
-VLC_API int64_t vlc_linear_split_workspace(int64_t rows, int64_t out_features) {
+VLC_API int vlc_linear_skinny_silu(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
+                                   const void* weight, int64_t w_row_stride, int64_t inter, void* out,
+                                   int64_t out_row_stride, void* stream) {
+  using namespace vlc;
+  const int bad = check(x, x_row_stride, rows, kMaxRows, in_features, weight, w_row_stride, inter, nullptr, out,
+                        out_row_stride);
+  if (bad != VLC_OK || rows == 0) return bad;
+  const Args a = {static_cast<const char*>(x), x_row_stride * 2, (int)rows, 0, 0, static_cast<const char*>(weight),
+                  w_row_stride * 2, nullptr, static_cast<uint16_t*>(out), out_row_stride, nullptr, (int)inter};
+  hipStream_t st = as_stream(stream);
+  const int64_t k = in_features;
+  // as vlc_linear_skinny chooses for many features, with an even number of feature groups
+  if (rows <= 2 && k % 256 == 0)
+    launch<2, 4, 8, 2, 1, 4, true>(a, k, 1, st);
+  else if (rows <= 4 && k % 128 == 0)
+    launch<2, 8, 4, 4, 1, 8, true>(a, k, 1, st);
+  else if (rows <= 8 && k % 64 == 0)
+    launch<2, 4, 2, 4, 1, 4, true>(a, k, 1, st);
+  else if (k % 64 == 0)
+    launch<2, 4, 2, 4, 2, 4, true>(a, k, 1, st);
+  else
+    launch<2, 8, 1, 2, 1, 8, true>(a, k, 1, st);
+  return launch_status();
+}
+
+VLC_API int64_t vlc_linear_split_workspace(int64_t rows, int64_t in_features, int64_t out_features) {
   using namespace vlc;
   if (rows <= 0 || rows > kMaxSplitRows || out_features < 32 || out_features >= ((int64_t)1 << 24)) return 0;
-  return num_splits(out_features) * rows * out_features * 4;
+  return num_splits(out_features / split_tile(rows, in_features, out_features)) * rows * out_features * 4;
 }
 
 VLC_API int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
@@ -232,9 +281,9 @@ VLC_API int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, 
                         out, out_row_stride);
   if (bad != VLC_OK || rows == 0) return bad;
   if (out_features % 32 || out_features >= ((int64_t)1 << 24)) return VLC_ERR_UNSUPPORTED;
-  const int splits = num_splits(out_features);
+  const int tile = split_tile(rows, in_features, out_features), splits = num_splits(out_features / tile);
   if (splits > 1 && (!workspace || !aligned16(workspace) ||
-                     workspace_bytes < vlc_linear_split_workspace(rows, out_features)))
+                     workspace_bytes < vlc_linear_split_workspace(rows, in_features, out_features)))
     return VLC_ERR_WORKSPACE;
   const Args a = {static_cast<const char*>(x), x_row_stride * 2, (int)rows, 0, 0, static_cast<const char*>(weight),
                   w_row_stride * 2, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(out), out_row_stride,
@@ -242,12 +291,24 @@ VLC_API int vlc_linear_split(const void* x, int64_t x_row_stride, int64_t rows, 
   hipStream_t st = as_stream(stream);
   if (rows <= 16)
     launch<2, 4, 1, 2, 1, 4>(a, in_features, splits, st);
-  else if (rows <= 32)
+  else if (rows <= 32 && in_features % 64 == 0) {
+    if (tile == 64)
+      launch<2, 4, 2, 8, 4, 4>(a, in_features, splits, st);
+    else
+      launch<1, 8, 2, 4, 4, 8>(a, in_features, splits, st);
+  } else if (rows <= 32)
     launch<2, 4, 1, 2, 2, 4>(a, in_features, splits, st);
-  else if (rows <= 48)
-    launch<2, 4, 1, 2, 3, 4>(a, in_features, splits, st);
-  else
-    launch<2, 4, 1, 2, 4, 4>(a, in_features, splits, st);
+  else if (rows <= 48) {
+    if (tile == 64)
+      launch<2, 4, 1, 4, 3, 4>(a, in_features, splits, st);
+    else
+      launch<2, 4, 1, 2, 3, 4>(a, in_features, splits, st);
+  } else {
+    if (tile == 64)
+      launch<2, 4, 1, 4, 4, 4>(a, in_features, splits, st);
+    else
+      launch<2, 4, 1, 2, 4, 4>(a, in_features, splits, st);
+  }
   const int st1 = launch_status();
   if (st1 != VLC_OK || splits == 1) return st1;
   const int64_t lanes = rows * out_features / 4;

@@ -800,6 +800,25 @@ def linear_skinny(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
     return out
 
 
+def linear_skinny_silu_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether vlc_linear_skinny_silu takes this call (as linear_skinny_supported, 16 | inter)."""
+    return _few_rows_supported(x, weight, None, SKINNY_MAX_ROWS) and weight.shape[0] % 32 == 0
+
+
+def linear_skinny_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of x [M <= 16, K] @ weight [2 * inter, K]^T (vlc_linear_skinny_silu) -> [M, inter]."""
+    _require_device("linear_skinny_silu", x, weight)
+    if not linear_skinny_silu_supported(x, weight):
+        raise ValueError(f"linear_skinny_silu does not take x {tuple(x.shape)} / weight {tuple(weight.shape)}")
+    m, k = x.shape
+    inter = weight.shape[0] // 2
+    out = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)
+    st = _lib.load().vlc_linear_skinny_silu(x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0),
+                                            inter, out.data_ptr(), inter, _stream(x))
+    _lib.check("vlc_linear_skinny_silu", st)
+    return out
+
+
 def linear_split_supported(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
     """Whether vlc_linear_split takes this call (as linear_skinny_supported, at most 64 rows, N % 32)."""
     return _few_rows_supported(x, weight, bias, SPLIT_MAX_ROWS) and weight.shape[0] % 32 == 0
@@ -815,7 +834,7 @@ def linear_split(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     n = weight.shape[0]
     lib = _lib.load()
     out = torch.empty(m, n, dtype=torch.bfloat16, device=x.device)
-    ws = torch.empty(lib.vlc_linear_split_workspace(m, n), dtype=torch.uint8, device=x.device)
+    ws = torch.empty(lib.vlc_linear_split_workspace(m, k, n), dtype=torch.uint8, device=x.device)
     st = lib.vlc_linear_split(x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0), n,
                               bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
                               ws.data_ptr(), ws.numel(), _stream(x))

@@ -6,7 +6,7 @@ on one GPU) are plain linear layers; in a decode step they see one row per
 sequence, and streaming the weights is the whole cost.  Calls with at most 16
 rows that vlc_linear_skinny takes run there; calls of 17 to 64 rows on a weight at least
 four times as long as it is tall run in vlc_linear_split (the down projections: 18944 x 3584
-with 32 rows 43 us against the library's 110, 11008 x 2048 20 against 27; on the other
+with 32 rows 38 us against the library's 110, 11008 x 2048 18 against 27; on the other
 projections, where K is at most N, the library is the faster one from 17 rows on, 3584 x
 37888 57 against 82 us).  Every other call is torch's F.linear (hipBLASLt).
 """

@@ -10,8 +10,9 @@ GEMMs run on torch (hipBLASLt) except calls of at most 16 rows (decode steps),
 which stream the weights through vlc_linear_skinny (layers.linear.Linear); per layer the rotary
 embedding of q and k and the KV store run as one gfx950 kernel and the
 attention as another (layers.attention.Attention), each RMSNorm (with its
-residual add) as one kernel and the MLP's SiLU-and-multiply as one, or for many
-rows as the epilogue of its gate/up projection (vlc_linear_silu).
+residual add) as one kernel and the MLP's SiLU-and-multiply as one, or as the
+epilogue of its gate/up projection (vlc_linear_silu for many rows,
+vlc_linear_skinny_silu for a decode step's).
 When the model config carries a vision_config the model owns the vision tower
 (vision.VisionTransformer, the cold path behind the encoder cache).
 Weights are random N(0, 0.02) unless loaded by the caller.
@@ -76,9 +77,11 @@ class MLP(nn.Module):
 
     def forward(self, x):
         g = self.gate_up_proj
-        if x.dim() == 2 and kernels.linear_silu_pays(x.shape[0], self.inter) and g.bias is None and \
-                kernels.plain_linear(g) and kernels.linear_silu_supported(x, g.weight):
-            return self.down_proj(kernels.linear_silu(x, g.weight))
+        if x.dim() == 2 and g.bias is None and kernels.plain_linear(g):
+            if kernels.linear_skinny_silu_supported(x, g.weight):
+                return self.down_proj(kernels.linear_skinny_silu(x, g.weight))
+            if kernels.linear_silu_pays(x.shape[0], self.inter) and kernels.linear_silu_supported(x, g.weight):
+                return self.down_proj(kernels.linear_silu(x, g.weight))
         return self.down_proj(kernels.silu_mul(g(x)))
 
 
