@@ -189,7 +189,7 @@ __device__ __forceinline__ float half_wave_max(float x) {
 // every V row in LDS holds a one and zeros throughout, so dim 80 of O^T += V^T P^T is the row sum of
 // the probabilities: the 32 adds a tile that the VALU, which bounds 80-dim heads, would spend on it
 // ride on products that run over dims 64..95 anyway (fp32 sums of the bf16 P that also weigh V).  A 4K
-// image's whole-image block with it 12465 us, 13650 with the padded form, its rotary kernel (160 us a
+// image's whole-image block with it 11835 us (12465 before full tiles took fixed load offsets), 13650 with the padded form, its rotary kernel (160 us a
 // block against 80) and its unpadding copy (46 us); the error against 64 bits is the same.
 template <int MODE, int KS = 8, int MB = 4, bool AHEAD = false, bool PACKED = false>
 __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const Params p) {
@@ -301,6 +301,13 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
       asm volatile("" : "+s"(lanes[j]));  // kept in scalar registers
     }
   }
+  // PACKED: the lane's offsets within a full tile (q, k and v are parts of the same rows: one stride)
+  uint32_t row_off[4];
+  if constexpr (PACKED) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) row_off[j] = (lrow0 + 4 * j) * (uint32_t)kst + ((lchunk0 ^ (uint32_t)j) << 4);
+  }
+
   // ---- state ---------------------------------------------------------------------
   f32x16 o[4];
 #pragma unroll
@@ -452,9 +459,12 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
   // 3, one or two exp2 per unit after), so the VALU work fills the matrix pipe's
   // shadow.  P^T of tile t-1 is read by the PV MFMAs before the softmax packs the
   // new one after the last unit.
-  auto step_body = [&](auto masked, int t, f32x16 (&s_cur)[2], f32x16 (&s_nxt)[2], uint8_t* k_rd, uint8_t* v_rd,
+  // kind 0: every key of tile t is visible; 1: the mask is applied; 2 (PACKED): as 0, and K tile t + 2 is a
+  // full tile too, so the tile loads need no clamp of their rows and take the lane's fixed offsets.
+  auto step_body = [&](auto kind, int t, f32x16 (&s_cur)[2], f32x16 (&s_nxt)[2], uint8_t* k_rd, uint8_t* v_rd,
                        uint8_t* k_ld, uint8_t* v_ld) __attribute__((always_inline)) {
-    constexpr bool MASKED = decltype(masked)::value;
+    constexpr bool MASKED = decltype(kind)::value == 1;
+    constexpr bool FULL = decltype(kind)::value == 2;
     constexpr int kAhead = 3;
     const int kt = k_begin + t * kTileK;
     // kAheadSrc: the sources were computed a step ahead (reading the block ids here
@@ -462,8 +472,10 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
     // step's sources are computed in units kRawUnit (block id reads) and kSrcUnit.
     constexpr int kRawUnit = 8, kSrcUnit = 20;
     static_assert(!kAheadSrc || kSrcUnit < NU, "the next step's sources are computed inside the step");
-    const DmaSrc dk = kAheadSrc ? dk_cur : dma_src(t + 2, kcol, kst);
-    const DmaSrc dv = kAheadSrc ? dv_cur : dma_src(t, vcol, vst);
+    const DmaSrc dk = FULL ? DmaSrc{kcol + ((int64_t)k0 + kt + 2 * kTileK) * kst, kTileK - 1}
+                           : kAheadSrc ? dk_cur : dma_src(t + 2, kcol, kst);
+    const DmaSrc dv = FULL ? DmaSrc{vcol + ((int64_t)k0 + kt) * vst, kTileK - 1}
+                           : kAheadSrc ? dv_cur : dma_src(t, vcol, vst);
     int32_t raw_k = 0, raw_v = 0;
     const uint32_t lr = opaque(lrow0), lcn = opaque(lchunk0);
     const int rel = min(limit, k_end - 1) - kt - 4 * hf;  // MASKED: keys past rel are masked
@@ -528,7 +540,12 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
       if (i + kAhead < NU) read_op(i + kAhead);
       mfma_op(i);
       // row (< 64) x row stride (< 2^24 bytes, checked on the host): a 24-bit multiply-add
-      if constexpr (PACKED) {
+      if constexpr (FULL) {
+        if (i < 4)
+          dma16_lanes(lanes[i], dk.base, row_off[i], lds_u32(k_ld + (16 * wave + 4 * i) * 256));
+        else if (i < 8)
+          dma16_lanes(lanes[i - 4], dv.base, row_off[i - 4], lds_u32(v_ld + (16 * wave + 4 * (i - 4)) * 256));
+      } else if constexpr (PACKED) {
         if (i < 4) {
           dma16_lanes(lanes[i], dk.base, __umul24(min(lr + 4 * i, dk.last), (uint32_t)kst) + ((lcn ^ (uint32_t)i) << 4),
                       lds_u32(k_ld + (16 * wave + 4 * i) * 256));
@@ -602,16 +619,16 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
     rescale(alpha);
     sync_tiles();
   };
-  auto step = [&](auto par, auto masked, int t) __attribute__((always_inline)) {
+  auto step = [&](auto par, auto kind, int t) __attribute__((always_inline)) {
     if constexpr (decltype(par)::value != 0)
-      step_body(masked, t, s_odd, s_even, k_buf0, v_buf0, k_buf1, v_buf1);
+      step_body(kind, t, s_odd, s_even, k_buf0, v_buf0, k_buf1, v_buf1);
     else
-      step_body(masked, t, s_even, s_odd, k_buf1, v_buf1, k_buf0, v_buf0);
+      step_body(kind, t, s_even, s_odd, k_buf1, v_buf1, k_buf0, v_buf0);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  using Masked = std::integral_constant<bool, true>;
-  using Plain = std::integral_constant<bool, false>;
+  using Masked = std::integral_constant<int, 1>;
+  using Plain = std::integral_constant<int, PACKED ? 2 : 0>;
 
   // ---- prologue: V buffer 1 zeroed, K tiles 0 and 1, S^T of tile 0 ----------------
   if (n_tiles > 0) {
@@ -685,7 +702,9 @@ __global__ __launch_bounds__(kThreads, kBlocksPerCU) void attn_fwd_kernel(const 
       }
     };
     int t = 0;
-    for (; t + 1 < n_plain; t += 2) {
+    // PACKED: the pair's K tiles t + 2 and t + 3 are full as well (a step more kind would not fit the registers:
+    // the last full tiles take the masked steps)
+    for (; t + (PACKED ? 3 : 1) < n_plain; t += 2) {
       prio(t, std::false_type{});
       step(I0{}, Plain{}, t);
       prio(t + 1, std::true_type{});
