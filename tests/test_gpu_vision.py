@@ -419,3 +419,22 @@ def test_packed_attention_refuses_foreign_plans(dev):
         plan = kernels.plan_attention(cu, cu, heads, heads, hd, False, dev)
         with pytest.raises((RuntimeError, ValueError)):
             kernels.vision_attention(qkv, 16, 0.1, plan)
+
+
+def test_tower_with_listeners_equals_the_tower(dev):
+    """Hooks on some blocks (which then add their own MLP output) see each block's output and change
+    nothing beyond the rounding of that sum to bf16: per-row cosine >= 0.9999."""
+    grids = [(1, 8, 12), (1, 18, 30)]
+    say("vision tower: hooked blocks")
+    vt = _tower(TINY, ov.random_params(TINY, seed=31), dev)
+    pix = _pixels(grids, 32).to(dev)
+    plain = vt(pix, grids).float().cpu()
+    for listened in ([0], [1], [0, 1, 2]):
+        seen = []
+        handles = [vt.blocks[i].register_forward_hook(lambda m, a, out: seen.append(out.shape)) for i in listened]
+        hooked = vt(pix, grids).float().cpu()
+        for h in handles:
+            h.remove()
+        assert len(seen) == len(listened) and all(tuple(x) == (pix.shape[0], TINY["hidden_size"]) for x in seen)
+        cos, _, _ = row_cosines(hooked, plain)
+        assert float(cos.min()) >= 0.9999
