@@ -443,6 +443,22 @@ int vlc_linear_silu(const void* x, int64_t x_row_stride, int64_t rows, int64_t i
                     const void* weight, int64_t w_row_stride, int64_t inter, const void* bias,
                     void* out, int64_t out_row_stride, int64_t out_width, void* stream);
 
+/*
+ * Linear layer of some hundred to a few thousand rows with a long K (down projections in a prefill):
+ * out[m][n] = bf16(sum_k x[m][k] * weight[n][k] + bias[n]), K split across workgroups, fp32 partial sums
+ * added in a fixed order.  bias: bf16 [out_features] or NULL.  in_features % 64 == 0,
+ * out_features % 4 == 0, rows * out_features < 2^31; x and weight 16-byte aligned with row strides
+ * multiples of 8 elements and below 2^22; out and bias 8-byte aligned, out_row_stride a multiple of 4
+ * (VLC_ERR_UNSUPPORTED otherwise).  workspace: device scratch of at least
+ * vlc_linear_tiled_workspace(rows, in_features, out_features) bytes, 16-byte aligned, used by this call
+ * only; its contents before and after do not matter.
+ */
+int64_t vlc_linear_tiled_workspace(int64_t rows, int64_t in_features, int64_t out_features);
+int vlc_linear_tiled(const void* x, int64_t x_row_stride, int64_t rows, int64_t in_features,
+                     const void* weight, int64_t w_row_stride, int64_t out_features, const void* bias,
+                     void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes,
+                     void* stream);
+
 #ifdef __cplusplus
 }
 #endif

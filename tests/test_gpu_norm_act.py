@@ -336,3 +336,35 @@ def test_linear_skinny_silu(dev, m, k, inter):
     scale = (1 + gu[:, :inter].float().abs()) * (1 + gu[:, inter:].float().abs())
     assert ((out - ref).abs() <= 2.0 ** -6 * scale).all()
     assert float((out == ref).float().mean()) >= 0.98 or out.numel() < 200
+
+
+# Every tile kind (256 x 256; 128 x 128 with four stages; 128 x 128, two a CU), K ranges shorter than the ring,
+# one split and several, partial tiles in both directions.
+@pytest.mark.parametrize("m,k,n,bias", [(1, 64, 4, True), (65, 18944, 3584, False), (256, 11008, 2048, True),
+                                        (100, 256, 132, True), (129, 704, 2052, False), (300, 4096, 1024, True),
+                                        (640, 18944, 3584, False), (1247, 11008, 2048, False), (700, 1280, 4100, True),
+                                        (2500, 8192, 2048, False)])
+def test_linear_tiled(dev, m, k, n, bias):
+    """vlc_linear_tiled against the exact product, three calls on the same operands (the first sees cold
+    weights): one bf16 ulp plus the reordering of K fp32 terms (the bar of test_linear_skinny), and the same bits
+    each time; the layer takes it from 65 rows on."""
+    from vlcache_amd import kernels
+    from vlcache_amd.layers.linear import Linear
+
+    say(f"linear_tiled m={m} k={k} n={n} bias={bias}")
+    x, w = randn_bf16((m, k + 8), m + k).to(dev)[:, :k], randn_bf16((n, k), n + k, 0.05).to(dev)
+    b = randn_bf16((n,), 9).to(dev) if bias else None
+    ref = x.double() @ w.double().t() + (b.double() if bias else 0.0)
+    tol = ref.abs() * 2.0 ** -7 + ref.abs().max() * k * 2.0 ** -24
+    outs = [kernels.linear_tiled(x, w, b) for _ in range(3)]
+    for out in outs:
+        assert int(((out.double() - ref).abs() > tol).sum()) == 0
+        assert torch.equal(out, outs[0])
+    if 64 < m <= 2500 and k >= 4 * n:
+        lin = Linear(k, n, bias=bias, device=dev, dtype=torch.bfloat16)
+        with torch.no_grad():
+            lin.weight.copy_(w)
+            if bias:
+                lin.bias.copy_(b)
+            assert torch.equal(lin(x), outs[0])
+        assert lin(x).requires_grad

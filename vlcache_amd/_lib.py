@@ -60,6 +60,8 @@ SIGNATURES = {
     "vlc_linear_split_workspace": (i64, [i64, i64, i64]),
     "vlc_linear_split": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, vp, i64, vp]),
     "vlc_linear_silu": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, i64, vp]),
+    "vlc_linear_tiled_workspace": (i64, [i64, i64, i64]),
+    "vlc_linear_tiled": (i32, [vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, vp, i64, vp]),
     "vlc_attn_plan": (
         i32,
         [c_i32p, c_i32p, i32, i32, i32, i32, i32, i32, c_i32p, i64, c_i64p, c_i64p],

@@ -23,7 +23,7 @@ ARCH = "gfx950"
 
 HIP_SOURCES = ["store_kvcache.hip", "rope_store_kv.hip", "rerotate_kv.hip", "varlen_attn.hip", "decode_attn.hip",
                "vision_rope.hip", "vision_window.hip", "norm_act.hip", "linear_skinny.hip",
-               "linear_silu.hip"]
+               "linear_silu.hip", "linear_tiled.hip"]
 HOST_SOURCES = ["attn_plan.cpp", "capi.cpp"]
 
 # Device flags: gfx950 only; packed-fp32 instructions are disabled for all HIP code.

@@ -842,14 +842,43 @@ def linear_split(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     return out
 
 
-# --------------------------------------------------------------------------- gate/up projection
+# --------------------------------------------------------------------------- tiled products
+TILED_MAX_ROWS = 2500  # of the layers' route to vlc_linear_tiled
+
+
+def linear_tiled_supported(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
+    """Whether vlc_linear_tiled takes this call (bf16, K % 64, N % 4, aligned rows)."""
+    return _tiled_supported(x, weight, bias, 4) and x.shape[0] * weight.shape[0] < 1 << 31
+
+
+def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """x [M, K] @ weight[N, K]^T + bias for a long K (vlc_linear_tiled); fp32 partial sums, one rounding."""
+    _require_device("linear_tiled", x, weight, bias)
+    if not linear_tiled_supported(x, weight, bias):
+        raise ValueError(f"linear_tiled does not take x {tuple(x.shape)} / weight {tuple(weight.shape)}")
+    m, k = x.shape
+    n = weight.shape[0]
+    lib = _lib.load()
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    ws = torch.empty(lib.vlc_linear_tiled_workspace(m, k, n), dtype=torch.uint8, device=x.device)
+    st = lib.vlc_linear_tiled(x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0), n,
+                              bias.data_ptr() if bias is not None else None, out.data_ptr(), n,
+                              ws.data_ptr(), ws.numel(), _stream(x))
+    _lib.check("vlc_linear_tiled", st)
+    return out
+
+
 def linear_silu_supported(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
     """Whether vlc_linear_silu takes this call (bf16, K % 64, whole groups of 4 features, aligned rows)."""
+    return _tiled_supported(x, weight, bias, 8)
+
+
+def _tiled_supported(x, weight, bias, n_multiple: int) -> bool:
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2):
         return False
     k, n = x.shape[1], weight.shape[0]
     xs, ws = x.stride(), weight.stride()
-    if weight.shape[1] != k or k % 64 or n % 8 or xs[1] != 1 or ws[1] != 1 or xs[0] % 8 or ws[0] % 8:
+    if weight.shape[1] != k or k % 64 or n % n_multiple or xs[1] != 1 or ws[1] != 1 or xs[0] % 8 or ws[0] % 8:
         return False
     if xs[0] < k or ws[0] < k or max(xs[0], ws[0]) >= 1 << 22 or x.data_ptr() % 16 or weight.data_ptr() % 16:
         return False
