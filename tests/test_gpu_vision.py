@@ -438,3 +438,16 @@ def test_tower_with_listeners_equals_the_tower(dev):
         assert len(seen) == len(listened) and all(tuple(x) == (pix.shape[0], TINY["hidden_size"]) for x in seen)
         cos, _, _ = row_cosines(hooked, plain)
         assert float(cos.min()) >= 0.9999
+    seen = []
+    inner = vt.blocks[1].forward
+    vt.blocks[1].forward = lambda *a: (seen.append("block"), inner(*a))[1]
+    vt.merger.register_forward_pre_hook(lambda m, a: seen.append(len(a)))
+    cos, _, _ = row_cosines(vt(pix, grids).float().cpu(), plain)
+    assert float(cos.min()) >= 0.9999 and seen == ["block", 1]
+
+
+def test_tower_without_images(dev):
+    """No patches: no embeddings, no error (nothing is launched for an empty batch)."""
+    vt = _tower(dict(REAL, depth=2, fullatt_block_indexes=[1]), ov.random_params(dict(REAL, depth=2), seed=3), dev)
+    out = vt(torch.zeros(0, 1176, dtype=torch.bfloat16, device=dev), [])
+    assert tuple(out.shape) == (0, 2048)

@@ -1062,7 +1062,9 @@ VLC_API int vlc_vision_attn(const void* qkv, int64_t qkv_row_stride, int num_hea
   if (head_dim != kHeadDimNarrow) return VLC_ERR_UNSUPPORTED;
   const int64_t width = (int64_t)num_heads * kHeadDimNarrow;
   if (num_heads <= 0 || qkv_row_stride < 3 * width || num_tokens < 0) return VLC_ERR_INVALID;
-  if (!qkv || !plan_host || !plan_dev || plan_len < kHeaderInts) return VLC_ERR_PLAN;
+  if (num_tokens == 0) return VLC_OK;
+  if (!qkv) return VLC_ERR_INVALID;
+  if (!plan_host || !plan_dev || plan_len < kHeaderInts) return VLC_ERR_PLAN;
   if (plan_len < kHeaderInts + ((int64_t)plan_host[kPNumItems] + plan_host[kPNumCombine]) * kItemInts) return VLC_ERR_PLAN;
   for (int64_t i = 0; i < plan_host[kPNumItems]; ++i) {  // the boundaries the kernel reads and writes by
     const int32_t* v = plan_host + kHeaderInts + i * kItemInts;

@@ -885,10 +885,15 @@ def _tiled_supported(x, weight, bias, n_multiple: int) -> bool:
     return bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 8 == 0)
 
 
+def no_listeners(m: torch.nn.Module) -> bool:
+    """Whether nobody hooked m's calls or replaced the instance's forward."""
+    return not (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__)
+
+
 def plain_linear(m: torch.nn.Module) -> bool:
     """Whether calling m is no more than its product: an nn.Linear without hooks, whose call a fused kernel
     may stand in for."""
-    return type(m).forward in _LINEAR_FORWARDS and not (m._forward_hooks or m._forward_pre_hooks)
+    return type(m).forward in _LINEAR_FORWARDS and no_listeners(m)
 
 
 _LINEAR_FORWARDS = {torch.nn.Linear.forward}  # layers.linear.Linear adds its own

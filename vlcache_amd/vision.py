@@ -301,11 +301,14 @@ class VisionTransformer(nn.Module):
         # 49 + 33), unless someone listens to the blocks' outputs
         delta = None
         for i, blk in enumerate(self.blocks):
-            if blk._forward_hooks or blk._forward_pre_hooks:
-                x, delta = blk(x if delta is None else x + delta, run, i in self.full), None
-            else:
+            if type(blk).forward is VisionBlock.forward and kernels.no_listeners(blk):
                 x, delta = blk.halves(x, delta, run, i in self.full)
-        return self.merger(x, delta).index_select(0, run.reverse)
+            else:
+                x, delta = blk(x if delta is None else x + delta, run, i in self.full), None
+        if type(self.merger).forward is not PatchMerger.forward or not kernels.no_listeners(self.merger):
+            x, delta = x if delta is None else x + delta, None
+        merged = self.merger(x) if delta is None else self.merger(x, delta)
+        return merged.index_select(0, run.reverse)
 
     @torch.no_grad()
     def load_checkpoint_weights(self, weights: dict) -> None:
