@@ -22,7 +22,8 @@
 // Measured, two window blocks of a 4K image (42196 patches, 16 heads): 4908 us for the tower
 // against 5474 us with the three passes (rotary into padded heads 160 us, attention of padded
 // heads 173 us, unpadding copy 46 us a block); eight blocks of a 64 x 64 image 2315 against 2524.
-// Windows of more than 64 patches take the three passes.
+// The kernel itself takes 102 us for the 432 MB (4.25 TB/s).  Larger windows are rotated in place
+// (vlc_vision_rope) and attend through vlc_vision_attn.
 #include "common.h"
 
 namespace vlc {
